@@ -411,103 +411,204 @@ __device__ inline uint64_t mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-constexpr int kLd = 65;  // padded row stride (conflict-free column access)
+// Row stride of the 64-wide LDS matrices of k_mlp_grad: a multiple of four
+// floats (16-byte reads) that spreads the rows over the banks.
+constexpr int kGs = kMlpH + 4;
+constexpr int kGt = 256;  // threads of a gradient block: a 4x4 output tile each
 
-// One sample per lane (kGradBlock lanes).  partial[block] receives this
-// block's gradient sums (kMlpNP floats) and loss sum.
-__global__ __launch_bounds__(kGradBlock) void k_mlp_grad(const float* __restrict__ P,
-                                                         const float* __restrict__ feats,
-                                                         const float* __restrict__ targets,
-                                                         uint64_t n, uint32_t count,
-                                                         uint64_t seed, float tau, float norm,
-                                                         float* __restrict__ partial) {
-  __shared__ float sW1[kMlpH][kMlpF + 1];
-  __shared__ float sW2[kMlpH][kLd];
+// 4x4 tile of a product summed over k in order: acc[i][j] += A[k][ia + i] *
+// B[k][jb + j] for k = 0 .. n-1, each multiply and add rounded on its own
+// (rows of A and B are kGs floats apart, 16-byte aligned).
+__device__ inline void tile_mac(const float* A, const float* B, int ia, int jb, int n,
+                                float (&acc)[4][4]) {
+#pragma unroll 4
+  for (int k = 0; k < n; ++k) {
+    const float4 a = *reinterpret_cast<const float4*>(A + k * kGs + ia);
+    const float4 b = *reinterpret_cast<const float4*>(B + k * kGs + jb);
+    const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] += av[i] * bv[j];
+  }
+}
+
+// Tile to row-major M[i][j] and, transposed, to MT[j][i] (nullable).
+__device__ inline void tile_store(const float (&v)[4][4], int i0, int j0, float* M, float* MT) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<float4*>(M + (i0 + i) * kGs + j0) =
+        make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
+  if (MT)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<float4*>(MT + (j0 + j) * kGs + i0) =
+          make_float4(v[0][j], v[1][j], v[2][j], v[3][j]);
+}
+
+// kGradBlock samples per block.  partial[block] receives this block's gradient
+// sums (kMlpNP floats) and loss sum.
+//
+// The five products of a block (two forward, one back, two weight gradients:
+// about 2M multiplies and adds) are FP32 VALU work in a fixed summation order,
+// so the network does not depend on how they are split.  A block holds every
+// matrix in LDS in the order its product reads it and each of 256 threads
+// takes 4x4 output tiles (two 16-byte LDS reads for 32 VALU operations).  One
+// sample per lane (64 threads, a scalar LDS read per operand) took 161 us
+// for a batch of 4096 (64 blocks); this form 36 us.
+__global__ __launch_bounds__(kGt) void k_mlp_grad(const float* __restrict__ P,
+                                                  const float* __restrict__ feats,
+                                                  const float* __restrict__ targets, uint64_t n,
+                                                  uint32_t count, uint64_t seed, float tau,
+                                                  float norm, float* __restrict__ partial) {
+  // Each matrix is named for what it holds first; mA holds gelu(z2) [s][o]
+  // after layer 2, mC the first layer's deltas [s][i] after the back product.
+  __shared__ __align__(16) float mA[kMlpH * kGs];   // W2^T [i][o]
+  __shared__ __align__(16) float mB[kMlpH * kGs];   // W2 [o][i]
+  __shared__ __align__(16) float mC[kMlpH * kGs];   // h1^T [i][s], h1 = bf16(gelu(z1))
+  __shared__ __align__(16) float mD[kMlpH * kGs];   // h1 [s][i]
+  __shared__ __align__(16) float mE[kMlpH * kGs];   // layer 2's deltas [s][o]
+  __shared__ __align__(16) float mF[kMlpH * kGs];   // the same transposed
+  __shared__ __align__(16) float mX[kGradBlock * kGs];  // x [s][f] (kMlpFP columns used)
+  __shared__ __align__(16) float mXT[kMlpF * kGs];  // x^T [f][s]
+  __shared__ __align__(16) float mW1[kMlpF * kGs];  // W1^T [f][o]
   __shared__ float sB1[kMlpH], sB2[kMlpH], sW3[kMlpH];
-  __shared__ float sX[kGradBlock][kMlpF + 1];
-  __shared__ float sZ1[kGradBlock][kLd];
-  __shared__ float sH1[kGradBlock][kLd];  // bf16(gelu(z1)), the input of layer 2
-  __shared__ float sZ2[kGradBlock][kLd];
-  __shared__ float sD2[kGradBlock][kLd];
-  __shared__ float sD1[kGradBlock][kLd];
-  __shared__ float sG[kGradBlock];
-  __shared__ float sLoss[kGradBlock];
+  __shared__ float sG[kGradBlock], sLoss[kGradBlock];
+  static_assert(kGradBlock == kMlpH && kGt == (kMlpH / 4) * (kMlpH / 4), "one tile per thread");
   const int t = threadIdx.x;
 
-  for (int i = t; i < kMlpH * kMlpF; i += kGradBlock) sW1[i / kMlpF][i % kMlpF] = round_bf(P[kOW1 + i]);
-  for (int i = t; i < kMlpH * kMlpH; i += kGradBlock) sW2[i / kMlpH][i % kMlpH] = round_bf(P[kOW2 + i]);
-  sB1[t] = P[kOB1 + t];
-  sB2[t] = P[kOB2 + t];
-  sW3[t] = round_bf(P[kOW3 + t]);
+  for (int i = t; i < kMlpH * kMlpF; i += kGt)
+    mW1[(i % kMlpF) * kGs + i / kMlpF] = round_bf(P[kOW1 + i]);
+  for (int i = t; i < kMlpH * kMlpH; i += kGt) {
+    const float w = round_bf(P[kOW2 + i]);
+    mB[(i / kMlpH) * kGs + i % kMlpH] = w;
+    mA[(i % kMlpH) * kGs + i / kMlpH] = w;
+  }
+  if (t < kMlpH) {
+    sB1[t] = P[kOB1 + t];
+    sB2[t] = P[kOB2 + t];
+    sW3[t] = round_bf(P[kOW3 + t]);
+  }
   const float b3 = P[kOB3];
+  // Sample s of the block: row of the feature table (four threads a sample,
+  // eight features each).
+  const auto sample_row = [&](int s, bool& valid) -> uint64_t {
+    const uint32_t si = blockIdx.x * kGradBlock + (uint32_t)s;
+    valid = si < count;
+    uint64_t row = si;
+    if (seed) row = mix64(seed ^ ((uint64_t)si * 0x100000001b3ull)) % n;
+    return row;
+  };
+  {
+    const int s = t / 4, f0 = 8 * (t % 4);
+    bool valid;
+    const uint64_t row = sample_row(s, valid);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int f = f0 + j;
+      const float v = valid && f < kMlpF ? round_bf(feats[row * kMlpFP + f]) : 0.0f;
+      mX[s * kGs + f] = v;
+      if (f < kMlpF) mXT[f * kGs + s] = v;
+    }
+  }
   __syncthreads();
 
-  const uint32_t si = blockIdx.x * kGradBlock + t;
-  const bool valid = si < count;
-  uint64_t row = si;
-  if (seed) row = mix64(seed ^ ((uint64_t)si * 0x100000001b3ull)) % n;
-  float x[kMlpF];
+  // Tile of this thread in every product: rows r0 .. r0+3, columns c0 .. c0+3.
+  const int r0 = 4 * (t % 16), c0 = 4 * (t / 16);
+  // forward: z1 [s][o], h1
+  float z1[4][4] = {};
+  tile_mac(mXT, mW1, r0, c0, kMlpF, z1);
+  {
+    float h[4][4];
 #pragma unroll
-  for (int f = 0; f < kMlpF; ++f) {
-    x[f] = valid ? round_bf(feats[row * kMlpFP + f]) : 0.0f;
-    sX[t][f] = x[f];
-  }
-  // forward
-  for (int o = 0; o < kMlpH; ++o) {
-    float z = 0.0f;
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int f = 0; f < kMlpF; ++f) z += sW1[o][f] * x[f];
-    z += sB1[o];
-    sZ1[t][o] = z;
-    sH1[t][o] = round_bf(gelu(z));
+      for (int j = 0; j < 4; ++j) {
+        z1[i][j] += sB1[c0 + j];
+        h[i][j] = round_bf(gelu(z1[i][j]));
+      }
+    tile_store(h, r0, c0, mD, mC);
   }
-  for (int o = 0; o < kMlpH; ++o) {
-    float z = 0.0f;
-    for (int i = 0; i < kMlpH; ++i) z += sW2[o][i] * sH1[t][i];
-    sZ2[t][o] = z + sB2[o];
+  __syncthreads();
+  // z2 [s][o]
+  float z2[4][4] = {};
+  tile_mac(mC, mA, r0, c0, kMlpH, z2);
+  __syncthreads();
+  {
+    float g2[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        z2[i][j] += sB2[c0 + j];
+        g2[i][j] = gelu(z2[i][j]);
+      }
+    tile_store(g2, r0, c0, mA, nullptr);
   }
-  float out = 0.0f;
-  for (int o = 0; o < kMlpH; ++o) out += sW3[o] * gelu(sZ2[t][o]);
-  out += b3;
-  const float tgt = valid ? targets[row] : 0.0f;
-  const float diff = tgt - out;
-  const float loss = valid ? (diff >= 0.0f ? tau * diff : (tau - 1.0f) * diff) : 0.0f;
-  const float g = valid ? norm * (out > tgt ? (1.0f - tau) : (out < tgt ? -tau : 0.0f)) : 0.0f;
-  sG[t] = g;
-  sLoss[t] = loss;
+  __syncthreads();
+  if (t < kGradBlock) {
+    bool valid;
+    const uint64_t row = sample_row(t, valid);
+    const float tgt = valid ? targets[row] : 0.0f;
+    float out = 0.0f;
+    for (int o = 0; o < kMlpH; ++o) out += sW3[o] * mA[t * kGs + o];
+    out += b3;
+    const float diff = tgt - out;
+    sLoss[t] = valid ? (diff >= 0.0f ? tau * diff : (tau - 1.0f) * diff) : 0.0f;
+    sG[t] = valid ? norm * (out > tgt ? (1.0f - tau) : (out < tgt ? -tau : 0.0f)) : 0.0f;
+  }
+  __syncthreads();
   // backward through layer 3 and 2
-  for (int o = 0; o < kMlpH; ++o) sD2[t][o] = g * sW3[o] * gelu_grad(sZ2[t][o]);
-  for (int i = 0; i < kMlpH; ++i) {
-    float d = 0.0f;
-    for (int o = 0; o < kMlpH; ++o) d += sW2[o][i] * sD2[t][o];
-    sD1[t][i] = d * gelu_grad(sZ1[t][i]);
+  {
+    float d2[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d2[i][j] = sG[r0 + i] * sW3[c0 + j] * gelu_grad(z2[i][j]);
+    tile_store(d2, r0, c0, mE, mF);
+  }
+  __syncthreads();
+  {
+    float d1[4][4] = {};
+    tile_mac(mF, mB, r0, c0, kMlpH, d1);  // [s][i]
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d1[i][j] = d1[i][j] * gelu_grad(z1[i][j]);
+    tile_store(d1, r0, c0, mC, nullptr);
   }
   __syncthreads();
 
-  // weight gradients: lane t owns output unit t of every layer
+  // weight gradients, summed over the samples in order
   float* dst = partial + (uint64_t)blockIdx.x * (kMlpNP + 1);
   {
-    float gb2 = 0.0f, gw3 = 0.0f, gb1 = 0.0f;
-    for (int s = 0; s < kGradBlock; ++s) {
-      gb2 += sD2[s][t];
-      gb1 += sD1[s][t];
-      gw3 += sG[s] * gelu(sZ2[s][t]);
-    }
-    dst[kOB2 + t] = gb2;
-    dst[kOB1 + t] = gb1;
-    dst[kOW3 + t] = gw3;
-    for (int i = 0; i < kMlpH; ++i) {
-      float acc = 0.0f;
-      for (int s = 0; s < kGradBlock; ++s) acc += sD2[s][t] * sH1[s][i];
-      dst[kOW2 + t * kMlpH + i] = acc;
-    }
-    for (int f = 0; f < kMlpF; ++f) {
-      float acc = 0.0f;
-      for (int s = 0; s < kGradBlock; ++s) acc += sD1[s][t] * sX[s][f];
-      dst[kOW1 + t * kMlpF + f] = acc;
-    }
+    float w2[4][4] = {};
+    tile_mac(mE, mD, c0, r0, kGradBlock, w2);  // [o][i]: rows c0.., columns r0..
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dst[kOW2 + (c0 + i) * kMlpH + r0 + j] = w2[i][j];
   }
-  if (t == 0) {
+  if (t % 16 < kMlpFP / 4) {
+    float w1[4][4] = {};
+    tile_mac(mC, mX, c0, r0, kGradBlock, w1);  // [o][f]
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (r0 + j < kMlpF) dst[kOW1 + (c0 + i) * kMlpF + r0 + j] = w1[i][j];
+  }
+  const int w = t / kWave, l = t % kWave;
+  if (w < 3) {
+    float acc = 0.0f;
+    if (w == 0)
+      for (int s = 0; s < kGradBlock; ++s) acc += mE[s * kGs + l];
+    else if (w == 1)
+      for (int s = 0; s < kGradBlock; ++s) acc += mC[s * kGs + l];
+    else
+      for (int s = 0; s < kGradBlock; ++s) acc += sG[s] * mA[s * kGs + l];
+    dst[(w == 0 ? kOB2 : w == 1 ? kOB1 : kOW3) + l] = acc;
+  } else if (l == 0) {
     float gb3 = 0.0f, ls = 0.0f;
     for (int s = 0; s < kGradBlock; ++s) {
       gb3 += sG[s];
@@ -518,27 +619,44 @@ __global__ __launch_bounds__(kGradBlock) void k_mlp_grad(const float* __restrict
   }
 }
 
+// Sum over the blocks' partials of parameter p in block order.  The adds are
+// one serial chain, the loads are not: 16 are in flight at a time, in blocks of
+// one wave so that the 6209 parameters spread over 98 CUs (Adam step on 64
+// partials: 15.9 -> 4.8 us; loss over 1024 partials: 240 -> 29 us).
+__device__ inline float sum_partials(const float* __restrict__ partial, uint32_t nblocks,
+                                     uint32_t p) {
+  float s = 0.0f;
+  uint32_t b = 0;
+  for (; b + 16 <= nblocks; b += 16) {
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = partial[(uint64_t)(b + i) * (kMlpNP + 1) + p];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s += v[i];
+  }
+  for (; b < nblocks; ++b) s += partial[(uint64_t)b * (kMlpNP + 1) + p];
+  return s;
+}
+
 // grads[p] = sum over blocks of partial[b][p] (fixed order); loss likewise.
-__global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ partial,
+__global__ __launch_bounds__(kWave) void k_mlp_reduce(const float* __restrict__ partial,
                                                     uint32_t nblocks, float* __restrict__ grads,
                                                     float* __restrict__ loss) {
-  uint32_t p = blockIdx.x * 256 + threadIdx.x;
+  uint32_t p = blockIdx.x * kWave + threadIdx.x;
   if (p > (uint32_t)kMlpNP) return;
-  float s = 0.0f;
-  for (uint32_t b = 0; b < nblocks; ++b) s += partial[(uint64_t)b * (kMlpNP + 1) + p];
+  const float s = sum_partials(partial, nblocks, p);
   if (p < (uint32_t)kMlpNP) grads[p] = s;
   else if (loss) *loss = s;
 }
 
-__global__ __launch_bounds__(256) void k_mlp_adam(float* __restrict__ P, float* __restrict__ m,
+__global__ __launch_bounds__(kWave) void k_mlp_adam(float* __restrict__ P, float* __restrict__ m,
                                                   float* __restrict__ v,
                                                   const float* __restrict__ partial,
                                                   uint32_t nblocks, float lr, float bc1,
                                                   float bc2) {
-  uint32_t p = blockIdx.x * 256 + threadIdx.x;
+  uint32_t p = blockIdx.x * kWave + threadIdx.x;
   if (p >= (uint32_t)kMlpNP) return;
-  float g = 0.0f;
-  for (uint32_t b = 0; b < nblocks; ++b) g += partial[(uint64_t)b * (kMlpNP + 1) + p];
+  const float g = sum_partials(partial, nblocks, p);
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   float mm = b1 * m[p] + (1.0f - b1) * g;
   float vv = b2 * v[p] + (1.0f - b2) * g * g;
@@ -666,14 +784,14 @@ hipError_t mlp_grad(const MlpState& m, const float* feats, const float* targets,
                     hipStream_t st) {
   uint32_t nb = (count + kGradBlock - 1) / kGradBlock;
   if (nb == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(kGradBlock), 0, st, m.params, feats, targets, n,
+  hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(kGt), 0, st, m.params, feats, targets, n,
                      count, rand_seed, tau, norm, partial);
   return hipGetLastError();
 }
 
 hipError_t mlp_reduce(const float* partial, uint32_t nblocks, float* grads, float* loss,
                       hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks_for(kMlpNP + 1)), dim3(256), 0, st, partial,
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpNP + kWave) / kWave), dim3(kWave), 0, st, partial,
                      nblocks, grads, loss);
   return hipGetLastError();
 }
@@ -681,7 +799,7 @@ hipError_t mlp_reduce(const float* partial, uint32_t nblocks, float* grads, floa
 hipError_t mlp_adam(MlpState& m, uint32_t nblocks, float lr, int t, hipStream_t st) {
   float bc1 = 1.0f - std::pow(0.9f, (float)t);
   float bc2 = 1.0f - std::pow(0.999f, (float)t);
-  hipLaunchKernelGGL(k_mlp_adam, dim3(blocks_for(kMlpNP)), dim3(256), 0, st, m.params, m.adam_m,
+  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpNP + kWave - 1) / kWave), dim3(kWave), 0, st, m.params, m.adam_m,
                      m.adam_v, m.partial, nblocks, lr, bc1, bc2);
   return hipGetLastError();
 }
