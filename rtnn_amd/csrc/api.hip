@@ -8,6 +8,8 @@
 //   search kernel -> rows in original query order.
 #include <hip/hip_runtime.h>
 
+#include <float.h>
+
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -208,6 +210,7 @@ struct rtnn_ctx_s {
   // grid
   DevBuf keys, vals, counts, cell_start, spts, tmp, grids;
   DevBuf cboxes;  // hierarchical grids: bounding box per kChunkPts sorted points
+  DevBuf boxes;   // box tree of the packet walk
   GridDesc hgrid{};
   uint64_t ncells = 0;
   int sort_passes = 0;
@@ -262,7 +265,8 @@ struct rtnn_ctx_s {
     DevBuf* all[] = {&pts, &keys, &vals, &counts, &cell_start, &spts, &tmp, &grids,
                      &qin, &qkeys, &qvals, &qsorted, &oidx, &od2, &shortrows, &misc,
                      &tiles, &offs, &bboxes, &pgrid, &pcounts, &qradius, &tr_q, &tr_idx,
-                     &tr_d2, &tr_t, &tr_f, &tr_out, &bcnt, &boff, &bpairs, &cboxes, &ovf};
+                     &tr_d2, &tr_t, &tr_f, &tr_out, &bcnt, &boff, &bpairs, &cboxes, &ovf,
+                     &boxes};
     for (DevBuf* b : all) b->release();
     if (st3) (void)hipStreamSynchronize(st3);
     for (int i = 0; i < 2; ++i) {
@@ -313,6 +317,8 @@ int hip_fail(rtnn_ctx c, hipError_t e, const char* what) {
     hipError_t e_ = (expr);                                \
     if (e_ != hipSuccess) return hip_fail(ctx, e_, #expr); \
   } while (0)
+
+constexpr int kPacketKeyBits = 10;  // Morton bits per axis of the packet walk's points
 
 int bits_for(uint64_t maxval) {
   int b = 0;
@@ -494,6 +500,44 @@ int build_hgrid(rtnn_ctx ctx, float r, int want_levels) {
   return RTNN_OK;
 }
 
+// Box tree over ctx->pts for the packet walk: points in Morton order of a cubic
+// grid of 2^10 cells per axis over their box (the order only decides how
+// compact the boxes are, never a result).  *t describes it.
+int build_packet_tree(rtnn_ctx ctx, BoxTree* t) {
+  const uint64_t n = ctx->n;
+  GridDesc g;
+  std::memset(&g, 0, sizeof g);
+  float ext = 0.0f;
+  for (int a = 0; a < 3; ++a) {
+    g.mn[a] = ctx->bbox[a];
+    g.dim[a] = 1 << kPacketKeyBits;
+    ext = std::max(ext, std::min(ctx->bbox[a + 3] - ctx->bbox[a], FLT_MAX));
+  }
+  g.cell = ext > 0.0f ? ext / (float)(1 << kPacketKeyBits) : 1.0f;
+  g.inv = std::min(1.0f / g.cell, FLT_MAX);
+  g.npoints = (uint32_t)n;
+  g.morton = 2;
+  ctx->hgrid = g;
+  ctx->ncells = 0;
+  CK(ctx->grids.ensure(sizeof(GridDesc)));
+  CK(ctx->keys.ensure(4 * n));
+  CK(ctx->vals.ensure(4 * n));
+  CK(ctx->spts.ensure(16 * n + kSptsPadBytes));
+  CK(ctx->tmp.ensure(4 * radix_tmp_words(n)));
+  CK(ctx->boxes.ensure(32 * box_tree_layout(n, nullptr).boxes));
+  *t = box_tree_layout(n, ctx->boxes.as<float4>());
+  CK(cell_keys_single(ctx->pts.as<float>(), n, ctx->hgrid, ctx->grids.as<GridDesc>(),
+                      ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), ctx->st));
+  CK(hipEventRecord(ctx->ev_desc, ctx->st));
+  CK(radix_sort_pairs(ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), n, 3 * kPacketKeyBits,
+                      ctx->tmp.as<uint32_t>(), ctx->st, &ctx->sort_passes));
+  CK(build_box_tree(ctx->pts.as<float>(), ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(), *t,
+                    ctx->st));
+  ctx->spts_current = true;
+  ctx->hlevels = 0;
+  return RTNN_OK;
+}
+
 constexpr int kQueryKeyBits = 8;  // Morton bits per axis of the query order
 
 // Prepares queries in processing order (float4 with the output row in w).
@@ -502,7 +546,7 @@ constexpr int kQueryKeyBits = 8;  // Morton bits per axis of the query order
 // descriptors are on the device), so it overlaps the point sort on ctx->st;
 // ctx->st waits for it before returning work that reads *qproc.
 int prepare_queries(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
-                    const float4** qproc) {
+                    const float4** qproc, int key_bits = kQueryKeyBits) {
   if (!qxyz) {  // the points themselves, already in cell order
     *qproc = ctx->spts.as<float4>();
     return RTNN_OK;
@@ -527,11 +571,11 @@ int prepare_queries(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
     // queries still share their neighbourhood.
     int maxdim = std::max(ctx->hgrid.dim[0], std::max(ctx->hgrid.dim[1], ctx->hgrid.dim[2]));
     const int bits = bits_for((uint64_t)(maxdim - 1));
-    const int shift = std::max(0, bits - kQueryKeyBits);
+    const int shift = std::max(0, bits - key_bits);
     CK(query_morton_keys(dq, nq, ctx->grids.as<GridDesc>(), shift, ctx->qkeys.as<uint32_t>(),
                          ctx->qvals.as<uint32_t>(), s2));
     CK(radix_sort_pairs(ctx->qkeys.as<uint32_t>(), ctx->qvals.as<uint32_t>(), nq,
-                        3 * std::min(bits, kQueryKeyBits), ctx->tmp2.as<uint32_t>(), s2,
+                        3 * std::min(bits, key_bits), ctx->tmp2.as<uint32_t>(), s2,
                         nullptr));
   }
   CK(gather_points(dq, ctx->qvals.as<uint32_t>(), nq, ctx->qsorted.as<float4>(), s2));
@@ -853,12 +897,17 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
   CK(hipSetDevice(ctx->device));
   const bool timing = wait && (ctx->opt.time_stages != 0 || stats != nullptr);
   if (timing) CK(hipEventRecord(ctx->ev[0], ctx->st));
+  // KNN with one query per lane (k <= 64) walks the box tree in packets; queries
+  // left in input order (query_order = 1) make no packets and walk the cells.
+  const bool packet = mode == RTNN_MODE_KNN && gl == 1 && !pooled && ctx->opt.query_order != 1;
   float f = ctx->opt.cell_factor > 0 ? ctx->opt.cell_factor : default_cell_factor(mode);
-  rc = build_grid(ctx, r / f);
+  BoxTree tree{};
+  rc = packet ? build_packet_tree(ctx, &tree) : build_grid(ctx, r / f);
   if (rc) return rc;
   if (timing) CK(hipEventRecord(ctx->ev[1], ctx->st));
   const float4* qproc = nullptr;
-  rc = prepare_queries(ctx, qxyz, nq, on_device, &qproc);
+  rc = prepare_queries(ctx, qxyz, nq, on_device, &qproc,
+                       packet ? kPacketKeyBits : kQueryKeyBits);
   if (rc) return rc;
   if (timing) CK(hipEventRecord(ctx->ev[2], ctx->st));
   OutBufs o;
@@ -869,8 +918,11 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
     rc = arm_overflow(ctx, nq, a);
     if (rc) return rc;
   }
-  CK(launch_search(a, mode == RTNN_MODE_KNN, gl, ctx->st, ctx->num_cus, wide_buffers(ctx),
-                   tile_points(ctx), false, pooled ? ctx->opt.queries_per_wave : 0));
+  if (packet)
+    CK(launch_knn_packet(a, tree, ctx->st, ctx->num_cus));
+  else
+    CK(launch_search(a, mode == RTNN_MODE_KNN, gl, ctx->st, ctx->num_cus, wide_buffers(ctx),
+                     tile_points(ctx), false, pooled ? ctx->opt.queries_per_wave : 0));
   if (timing) CK(hipEventRecord(ctx->ev[3], ctx->st));
   rc = copy_out(ctx, nq, k, out_idx, out_d2, out_on_device, o);
   if (rc) return rc;

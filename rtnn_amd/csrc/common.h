@@ -26,7 +26,8 @@ struct GridDesc {
   uint32_t cell_base;   // first cell of this grid in the global cell table
   uint32_t point_base;  // first point of this cloud in the input order
   uint32_t npoints;
-  uint32_t morton;      // 1: cells numbered cell_base + Morton code (cubic grid)
+  uint32_t morton;      // 1: cells numbered cell_base + Morton code, 2: Hilbert key
+                        // (cubic grids)
 };
 static_assert(sizeof(GridDesc) == 48, "GridDesc layout");
 
@@ -89,6 +90,21 @@ struct SearchArgs {
   uint32_t* ovf_count;
 };
 
+// Box tree over the Morton-sorted points (packet.hip): leaves of kLeafPts
+// consecutive points, nodes of kFan children.  Level 0 holds the leaves' boxes
+// (minimum at box[2i], maximum at box[2i + 1]), level l + 1 those of kFan
+// consecutive boxes of level l; the top level has at most kFan.
+constexpr int kLeafPts = 8;
+constexpr int kFan = 64;
+constexpr int kTreeLevels = 6;  // 8 * 64^5 points: more than 2^32
+struct BoxTree {
+  const float4* box;
+  uint32_t off[kTreeLevels];  // first box of each level
+  uint32_t cnt[kTreeLevels];  // its boxes
+  int top;
+  uint64_t boxes;  // of all levels
+};
+
 constexpr uint32_t kTreeLeafDefault = 256;
 
 constexpr uint32_t kChunkPts = 32;
@@ -138,6 +154,31 @@ __host__ __device__ inline uint32_t spread3(uint32_t x) {
 }
 __host__ __device__ inline uint32_t morton3(uint32_t x, uint32_t y, uint32_t z) {
   return (spread3(z) << 2) | (spread3(y) << 1) | spread3(x);
+}
+
+// Position of a cell (10-bit coordinates) on the Hilbert curve of a 2^10 cubic
+// grid, 30 bits: Skilling's transform of the axes to the transposed index
+// ("Programming the Hilbert curve", AIP Conf. Proc. 707, 2004), interleaved.
+// Consecutive keys are neighbouring cells, where a Morton key jumps.
+__host__ __device__ inline uint32_t hilbert3(uint32_t x, uint32_t y, uint32_t z) {
+#pragma unroll
+  for (uint32_t q = 512u; q > 1u; q >>= 1) {
+    const uint32_t p = q - 1u;
+    // axis by axis: invert x's low bits, or exchange them with the axis's
+    x ^= (x & q) ? p : 0u;
+    const uint32_t ty = (y & q) ? 0u : (x ^ y) & p;
+    x ^= (y & q) ? p : ty;
+    y ^= ty;
+    const uint32_t tz = (z & q) ? 0u : (x ^ z) & p;
+    x ^= (z & q) ? p : tz;
+    z ^= tz;
+  }
+  y ^= x;
+  z ^= y;
+  uint32_t t = 0;
+#pragma unroll
+  for (uint32_t q = 512u; q > 1u; q >>= 1) t ^= (z & q) ? q - 1u : 0u;
+  return morton3(z ^ t, y ^ t, x ^ t);  // x's bit leads
 }
 
 // (d2, index) packed so unsigned 64-bit order is the lexicographic order

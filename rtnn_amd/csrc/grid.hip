@@ -304,8 +304,9 @@ __global__ __launch_bounds__(256) void k_cell_keys1(const float* __restrict__ xy
   const int cx = cell_of(xyz[3 * i], g.mn[0], g.inv, g.dim[0]);
   const int cy = cell_of(xyz[3 * i + 1], g.mn[1], g.inv, g.dim[1]);
   const int cz = cell_of(xyz[3 * i + 2], g.mn[2], g.inv, g.dim[2]);
-  keys[i] = g.cell_base + ((uint32_t)cz * (uint32_t)g.dim[1] + (uint32_t)cy) * (uint32_t)g.dim[0] +
-            (uint32_t)cx;
+  keys[i] = g.morton ? hilbert3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz)
+                     : g.cell_base + ((uint32_t)cz * (uint32_t)g.dim[1] + (uint32_t)cy) *
+                                         (uint32_t)g.dim[0] + (uint32_t)cx;
   vals[i] = (uint32_t)i;
 }
 
@@ -564,7 +565,7 @@ __global__ __launch_bounds__(256) void k_query_morton(const float* __restrict__ 
   uint32_t cx = (uint32_t)cell_of(q[3 * i], g.mn[0], g.inv, g.dim[0]) >> shift;
   uint32_t cy = (uint32_t)cell_of(q[3 * i + 1], g.mn[1], g.inv, g.dim[1]) >> shift;
   uint32_t cz = (uint32_t)cell_of(q[3 * i + 2], g.mn[2], g.inv, g.dim[2]) >> shift;
-  keys[i] = morton3(cx, cy, cz);
+  keys[i] = g.morton == 2 ? hilbert3(cx, cy, cz) : morton3(cx, cy, cz);
   vals[i] = (uint32_t)i;
 }
 

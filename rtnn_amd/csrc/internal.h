@@ -109,6 +109,16 @@ hipError_t bucket_snap(float* qradius, uint32_t nq, float snap_r, float r, hipSt
 hipError_t launch_search(const SearchArgs& a, int knn_mode, int group_lanes, hipStream_t st,
                          int num_cus, bool wide = true, int tiled = 0, bool deep = false,
                          int pool = 0);
+// ---- packet.hip
+// Level layout of the box tree of n points over `box` (2 * boxes float4).
+BoxTree box_tree_layout(uint64_t n, float4* box);
+// spts[j] = (xyz[vals[j]], bits(vals[j])), filled to whole leaves with points
+// at infinity, and the boxes of every level.
+hipError_t build_box_tree(const float* xyz, const uint32_t* vals, uint64_t n, float4* spts,
+                          const BoxTree& t, hipStream_t st);
+// KNN (k <= 64) of a's queries over the box tree of a.spts.
+hipError_t launch_knn_packet(const SearchArgs& a, const BoxTree& t, hipStream_t st, int num_cus);
+
 // Every device / pinned allocation of the library (tracked for
 // rtnn_mem_stats; logged with RTNN_MEMSTAT set).
 hipError_t dev_alloc(void** p, size_t bytes);

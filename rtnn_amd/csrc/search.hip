@@ -29,6 +29,7 @@
 
 #include "common.h"
 #include "internal.h"
+#include "topk.h"
 
 namespace rtnn {
 
@@ -36,18 +37,6 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ inline uint64_t lanemask_lt64() {
-  const int lane = threadIdx.x & (kWave - 1);
-  return lane == 0 ? 0ull : (~0ull >> (kWave - lane));
-}
-
-// d2 < R2 as d2 <= r2_limit(R2): the float just below R2 (-1 for R2 <= 0,
-// FLT_MAX for +inf).  After a select the limit becomes the k-th key's d2:
-// ties with it are appended too and resolved by the (d2, index) rank.
-__device__ inline float r2_limit(float R2) {
-  return R2 > 0.0f ? __uint_as_float(__float_as_uint(R2) - 1u) : -1.0f;
 }
 
 // Resolves tile t into its query range and grid.
@@ -61,11 +50,6 @@ __device__ inline void tile_of(const SearchArgs& a, uint32_t nq, uint32_t t, uin
     q1 = min(q0 + a.tile_q, nq);
     gi = 0;
   }
-}
-
-// Query count of this launch (device-resident for the fallback pass).
-__device__ inline uint32_t launch_nq(const SearchArgs& a) {
-  return a.nq_dev ? *a.nq_dev : a.nq;
 }
 
 // Persistent launches walk tiles in XCD-contiguous chunks; plain launches map
@@ -90,33 +74,6 @@ struct TileIter {
     }
   }
 };
-
-// Appends the processing positions of short rows (fewer than k hits) with
-// one atomic per wave; a wave's entries stay together and in lane order, so
-// the re-run over the list keeps the Morton locality of the queries.
-__device__ inline void append_short(const SearchArgs& a, bool is_short, uint32_t qs,
-                                    uint32_t hits, float R) {
-  const uint64_t m = __ballot(is_short);
-  if (m == 0) return;
-  const int leader = __ffsll((unsigned long long)m) - 1;
-  uint32_t base = 0;
-  if ((int)(threadIdx.x & (kWave - 1)) == leader)
-    base = atomicAdd(a.short_count, (uint32_t)__popcll(m));
-  base = __shfl(base, leader, kWave);
-  if (is_short) {
-    const uint32_t pos = base + (uint32_t)__popcll(m & lanemask_lt64());
-    a.short_rows[pos] = qs;
-    if (a.short_hits) a.short_hits[pos] = hits;
-    if (a.radius_out) a.radius_out[qs] = R;
-  }
-}
-
-// Search radius of launch position qi (query qs).
-__device__ inline float query_radius(const SearchArgs& a, uint32_t qi, uint32_t qs) {
-  if (!a.qradius) return a.r;
-  const float sc = a.qsel_hits ? hit_scale(a.qsel_hits[qi], a.k) : a.qradius_scale;
-  return fminf(a.r, a.qradius[qs] * sc);
-}
 
 // Candidates loaded per lane before the first is tested (thread kernel;
 // group kernel: its G lanes share a query, so each lane takes more), and
