@@ -6,7 +6,7 @@
 // sort.cpp:535-612 uses for the counting sort of particles into cells.
 //
 // Radix sort, one 8-bit digit per pass, three kernels per pass:
-//   rs_hist    : per 4096-key tile, a digit histogram (LDS atomics), stored
+//   rs_hist    : per tile (1024 or 4096 keys), a digit histogram (LDS atomics), stored
 //                digit-major (row d = every tile's count of digit d);
 //   rs_rowscan : one block per digit scans its row (the tile's start within
 //                the digit) and writes the digit's total;
@@ -27,8 +27,6 @@ constexpr int kScanItems = 16;
 constexpr int kScanTile = kScanThreads * kScanItems;  // 4096
 
 constexpr int kRsThreads = 256;
-constexpr int kRsItems = 16;
-constexpr int kRsTile = kRsThreads * kRsItems;  // 4096
 constexpr int kRsWaves = kRsThreads / kWave;
 
 // ---------------------------------------------------------------- scan ----
@@ -152,11 +150,22 @@ hipError_t exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32_
 // get shorter and its LDS use cuts the blocks per CU.)
 constexpr int kRsDigit = 8;
 
+// Keys per thread of a tile.  Large arrays take 4096-key tiles (the longer a
+// tile's digit runs, the better its stores coalesce); smaller ones 1024-key
+// tiles, whose serial ranking is a quarter as long and which give every CU
+// some (four passes of a 30-bit sort, all launches: 100k keys 79 -> 66 us, 300k
+// 85 -> 72; at 1M keys 92 -> 102, so the line lies at half a million).
+constexpr int kRsItemsLarge = 16, kRsItemsSmall = 4;
+constexpr uint64_t kRsSmallMax = 1ull << 19;
+static int rs_items(uint64_t n) { return n <= kRsSmallMax ? kRsItemsSmall : kRsItemsLarge; }
+
+template <int kRsItems>
 __global__ __launch_bounds__(kRsThreads) void k_rs_hist(const uint32_t* __restrict__ keys,
                                                         uint64_t n, int shift, uint32_t lowmask,
                                                         uint32_t ntiles,
                                                         uint32_t* __restrict__ hist) {
   constexpr int NB = 1 << kRsDigit;
+  constexpr int kRsTile = kRsThreads * kRsItems;
   __shared__ uint32_t h[NB];
   for (int i = threadIdx.x; i < NB; i += kRsThreads) h[i] = 0;
   __syncthreads();
@@ -227,6 +236,7 @@ __device__ inline uint64_t lanemask_lt() {
   return lane == 0 ? 0ull : (~0ull >> (kWave - lane));
 }
 
+template <int kRsItems>
 __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, uint64_t n, int shift,
@@ -234,6 +244,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(
     const uint32_t* __restrict__ hist_scan, const uint32_t* __restrict__ totals) {
   constexpr int DB = kRsDigit;
   constexpr int NB = 1 << DB;
+  constexpr int kRsTile = kRsThreads * kRsItems;
   constexpr int PT = NB / kRsThreads;               // digits per thread in the digit scans
   constexpr int kWaveItems = kRsTile / kRsWaves;    // consecutive tile items of one wave
   __shared__ uint32_t s_keys[kRsTile];
@@ -348,7 +359,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(
 }
 
 uint64_t radix_tmp_words(uint64_t n) {
-  const uint64_t ntiles = (n + kRsTile - 1) / kRsTile;
+  const uint64_t tile = (uint64_t)kRsThreads * rs_items(n);
+  const uint64_t ntiles = (n + tile - 1) / tile;
   const uint64_t hist = (1ull << kRsDigit) * ntiles;
   // two key/value ping-pong buffers, raw and scanned tile histograms, totals
   return 4 * n + 2 * hist + (1ull << kRsDigit) + 64;
@@ -364,7 +376,9 @@ hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint64_t n, int bits
   if (passes_out) *passes_out = passes;
   if (n <= 1 || passes == 0) return hipSuccess;
   const uint32_t lowmask = bits >= 32 ? 0xffffffffu : ((1u << bits) - 1u);
-  const uint32_t ntiles = (uint32_t)((n + kRsTile - 1) / kRsTile);
+  const bool small = rs_items(n) == kRsItemsSmall;
+  const uint64_t tile = (uint64_t)kRsThreads * rs_items(n);
+  const uint32_t ntiles = (uint32_t)((n + tile - 1) / tile);
   const uint64_t hsz = (1ull << kRsDigit) * ntiles;
   uint32_t* bk[2] = {tmp, tmp + 2 * n};
   uint32_t* bv[2] = {tmp + n, tmp + 3 * n};
@@ -378,12 +392,13 @@ hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint64_t n, int bits
     uint32_t* kb = last ? keys : bk[p & 1];
     uint32_t* vb = last ? vals : bv[p & 1];
     const int shift = kRsDigit * p;
-    hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(kRsThreads), 0, st, ka, n, shift, lowmask,
-                       ntiles, hraw);
+    hipLaunchKernelGGL(small ? k_rs_hist<kRsItemsSmall> : k_rs_hist<kRsItemsLarge>, dim3(ntiles),
+                       dim3(kRsThreads), 0, st, ka, n, shift, lowmask, ntiles, hraw);
     hipLaunchKernelGGL(k_rs_rowscan, dim3(1u << kRsDigit), dim3(kScanThreads), 0, st, hraw,
                        ntiles, hscan, totals);
-    hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(kRsThreads), 0, st, ka, va, kb, vb, n,
-                       shift, lowmask, ntiles, hraw, hscan, totals);
+    hipLaunchKernelGGL(small ? k_rs_scatter<kRsItemsSmall> : k_rs_scatter<kRsItemsLarge>,
+                       dim3(ntiles), dim3(kRsThreads), 0, st, ka, va, kb, vb, n, shift, lowmask,
+                       ntiles, hraw, hscan, totals);
     ka = kb;
     va = vb;
   }
