@@ -110,7 +110,7 @@ typedef struct {
   uint64_t fallback_queries; /* rows short after the first stage (proposal search) */
   uint32_t grid_dims[3];
   float    cell_size;
-  uint32_t sort_passes;   /* LSD radix passes of the point sort                     */
+  uint32_t sort_passes;   /* LSD radix passes of the point sort (0: counted into cells) */
   uint32_t search_launches;
   uint32_t lanes_per_query; /* range kernel group width actually used               */
   double ms_copy;         /* result copy to host arrays (host outputs only)          */

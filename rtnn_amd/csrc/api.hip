@@ -209,6 +209,7 @@ struct rtnn_ctx_s {
 
   // grid
   DevBuf keys, vals, counts, cell_start, spts, tmp, grids;
+  uint64_t counts_zero = 0;  // leading words of `counts` known to be zero
   DevBuf cboxes;  // hierarchical grids: bounding box per kChunkPts sorted points
   DevBuf boxes;   // box tree of the packet walk
   GridDesc hgrid{};
@@ -384,9 +385,37 @@ int group_lanes_from_opt(rtnn_ctx ctx, int mode, uint32_t k) {
   return gl;
 }
 
+// Raster grids are built by counting up to a million points, by sorting beyond:
+// the counting build is a third of the launches, which is what a small grid
+// costs, but its atomics on random cells run at about 25 G/s, and its 16-byte
+// stores are scattered where the sort's gather reads are.  Build time by
+// counting / by sorting (uniform points, 0.2 cells per point): 50k 16 / 44 us,
+// 200k 31 / 50, 800k 63 / 95, 1.6M 106 / 124; sphere surfaces (8 cells per
+// point): 200k 32 / 64, 800k 84 / 110, 1.6M 155 / 154.  (10M points, 7 cells
+// each: 1390 against 780.)
+bool count_cells_rule(uint64_t n, uint64_t ncells) {
+  return n <= (1ull << 20) && ncells <= (1ull << 25);
+}
+
+// Makes the first ncells words of ctx->counts zero for a grid build.  The build
+// leaves them zero (grid_built), so they are cleared only when the table grows
+// or a build was cut short.
+int clear_counts(rtnn_ctx ctx, uint64_t ncells) {
+  const void* before = ctx->counts.p;
+  CK(ctx->counts.ensure(4 * ((ncells + 3) & ~3ull)));
+  if (ctx->counts.p != before) ctx->counts_zero = 0;
+  if (ctx->counts_zero < ncells) CK(fill_u32(ctx->counts.as<uint32_t>(), ncells, 0, ctx->st));
+  ctx->counts_zero = 0;
+  return RTNN_OK;
+}
+void grid_built(rtnn_ctx ctx, uint64_t ncells, uint64_t was_zero) {
+  ctx->counts_zero = std::max(ncells, was_zero);
+}
+
 // Builds the single-cloud grid over ctx->pts with edge `cell` (grown until the
-// cell count fits the budget).
-int build_grid(rtnn_ctx ctx, float cell) {
+// cell count fits the budget).  desc_event: separate queries follow, ordered on
+// the second stream as soon as the descriptor is on the device.
+int build_grid(rtnn_ctx ctx, float cell, bool desc_event = true) {
   GridDesc g;
   const uint64_t cap = max_cells_for(ctx, ctx->n);
   for (int tries = 0;; ++tries) {
@@ -406,19 +435,36 @@ int build_grid(rtnn_ctx ctx, float cell) {
   CK(ctx->vals.ensure(4 * n));
   CK(ctx->cell_start.ensure(4 * (ctx->ncells + 1)));
   CK(ctx->spts.ensure(16 * std::max<uint64_t>(n, 1) + kSptsPadBytes));
-  CK(ctx->tmp.ensure(4 * std::max(radix_tmp_words(n), cell_bounds_tmp_words(ctx->ncells))));
-  // The descriptor goes to the device as the key kernel's argument (no
-  // pageable copy, which costs the host more than a launch).
-  CK(cell_keys_single(ctx->pts.as<float>(), n, ctx->hgrid, ctx->grids.as<GridDesc>(),
-                      ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), ctx->st));
-  CK(hipEventRecord(ctx->ev_desc, ctx->st));
-  CK(radix_sort_pairs(ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), n,
-                      bits_for(ctx->ncells - 1), ctx->tmp.as<uint32_t>(), ctx->st,
-                      &ctx->sort_passes));
-  CK(cell_bounds(ctx->keys.as<uint32_t>(), n, (uint32_t)ctx->ncells,
-                 ctx->cell_start.as<uint32_t>(), ctx->tmp.as<uint32_t>(), ctx->st));
-  CK(gather_points(ctx->pts.as<float>(), ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(),
-                   ctx->st));
+  if (count_cells_rule(n, ctx->ncells)) {
+    CK(ctx->tmp.ensure(4 * cell_scan_tmp_words(ctx->ncells)));
+    const uint64_t zero = ctx->counts_zero;
+    const int rc = clear_counts(ctx, ctx->ncells);
+    if (rc) return rc;
+    CK(cell_count_single(ctx->pts.as<float>(), n, ctx->hgrid, ctx->grids.as<GridDesc>(),
+                         ctx->counts.as<uint32_t>(), ctx->keys.as<uint32_t>(),
+                         ctx->vals.as<uint32_t>(), ctx->st));
+    if (desc_event) CK(hipEventRecord(ctx->ev_desc, ctx->st));
+    CK(cell_scan_place(ctx->pts.as<float>(), n, ctx->ncells, ctx->counts.as<uint32_t>(),
+                       ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(),
+                       ctx->cell_start.as<uint32_t>(), ctx->tmp.as<uint32_t>(),
+                       ctx->spts.as<float4>(), ctx->st));
+    grid_built(ctx, ctx->ncells, zero);
+    ctx->sort_passes = 0;
+  } else {
+    CK(ctx->tmp.ensure(4 * std::max(radix_tmp_words(n), cell_bounds_tmp_words(ctx->ncells))));
+    // The descriptor goes to the device as the key kernel's argument (no
+    // pageable copy, which costs the host more than a launch).
+    CK(cell_keys_single(ctx->pts.as<float>(), n, ctx->hgrid, ctx->grids.as<GridDesc>(),
+                        ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), ctx->st));
+    if (desc_event) CK(hipEventRecord(ctx->ev_desc, ctx->st));
+    CK(radix_sort_pairs(ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), n,
+                        bits_for(ctx->ncells - 1), ctx->tmp.as<uint32_t>(), ctx->st,
+                        &ctx->sort_passes));
+    CK(cell_bounds(ctx->keys.as<uint32_t>(), n, (uint32_t)ctx->ncells,
+                   ctx->cell_start.as<uint32_t>(), ctx->tmp.as<uint32_t>(), ctx->st));
+    CK(gather_points(ctx->pts.as<float>(), ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(),
+                     ctx->st));
+  }
   ctx->spts_current = true;
   ctx->hlevels = 0;
   return RTNN_OK;
@@ -902,7 +948,7 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
   const bool packet = mode == RTNN_MODE_KNN && gl == 1 && !pooled && ctx->opt.query_order != 1;
   float f = ctx->opt.cell_factor > 0 ? ctx->opt.cell_factor : default_cell_factor(mode);
   BoxTree tree{};
-  rc = packet ? build_packet_tree(ctx, &tree) : build_grid(ctx, r / f);
+  rc = packet ? build_packet_tree(ctx, &tree) : build_grid(ctx, r / f, qxyz != nullptr);
   if (rc) return rc;
   if (timing) CK(hipEventRecord(ctx->ev[1], ctx->st));
   const float4* qproc = nullptr;
@@ -1894,17 +1940,32 @@ int build_batched(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets, uint3
   CK(ctx->vals.ensure(4 * n));
   CK(ctx->cell_start.ensure(4 * (total + 1)));
   CK(ctx->spts.ensure(16 * n + kSptsPadBytes));
-  CK(ctx->tmp.ensure(4 * std::max(radix_tmp_words(n), cell_bounds_tmp_words(total))));
   ctx->spts_current = false;  // spts now holds the clouds, not ctx->pts
   ctx->hlevels = 0;           // and grids/cell_start the clouds' raster grids
-  CK(cell_keys(xyz, n, ctx->grids.as<GridDesc>(), ctx->offs.as<uint64_t>(), nclouds,
-               ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), nullptr, ctx->st));
-  CK(radix_sort_pairs(ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), n,
-                      bits_for(total - 1), ctx->tmp.as<uint32_t>(), ctx->st,
-                      &ctx->sort_passes));
-  CK(cell_bounds(ctx->keys.as<uint32_t>(), n, (uint32_t)total, ctx->cell_start.as<uint32_t>(),
-                 ctx->tmp.as<uint32_t>(), ctx->st));
-  CK(gather_points(xyz, ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(), ctx->st));
+  if (count_cells_rule(n, total)) {
+    CK(ctx->tmp.ensure(4 * cell_scan_tmp_words(total)));
+    const uint64_t zero = ctx->counts_zero;
+    const int rc = clear_counts(ctx, total);
+    if (rc) return rc;
+    CK(cell_count(xyz, n, ctx->grids.as<GridDesc>(), ctx->offs.as<uint64_t>(), nclouds,
+                  ctx->counts.as<uint32_t>(), ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(),
+                  ctx->st));
+    CK(cell_scan_place(xyz, n, total, ctx->counts.as<uint32_t>(), ctx->keys.as<uint32_t>(),
+                       ctx->vals.as<uint32_t>(), ctx->cell_start.as<uint32_t>(),
+                       ctx->tmp.as<uint32_t>(), ctx->spts.as<float4>(), ctx->st));
+    grid_built(ctx, total, zero);
+    ctx->sort_passes = 0;
+  } else {
+    CK(ctx->tmp.ensure(4 * std::max(radix_tmp_words(n), cell_bounds_tmp_words(total))));
+    CK(cell_keys(xyz, n, ctx->grids.as<GridDesc>(), ctx->offs.as<uint64_t>(), nclouds,
+                 ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), nullptr, ctx->st));
+    CK(radix_sort_pairs(ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), n,
+                        bits_for(total - 1), ctx->tmp.as<uint32_t>(), ctx->st,
+                        &ctx->sort_passes));
+    CK(cell_bounds(ctx->keys.as<uint32_t>(), n, (uint32_t)total, ctx->cell_start.as<uint32_t>(),
+                   ctx->tmp.as<uint32_t>(), ctx->st));
+    CK(gather_points(xyz, ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(), ctx->st));
+  }
 
   // Tiles: runs of <= kTileQ sorted queries inside one cloud.  Cell keys are
   // cloud-major, so cloud c's points occupy sorted positions
@@ -2590,7 +2651,8 @@ struct rtnn_graph_s {
   hipGraphExec_t exec = nullptr;
   // Buffers owned by the graph, so calls on the context between replays
   // cannot move memory the graph's nodes point at.
-  DevBuf offs, bboxes, status, grids, keys, vals, cell_start, spts, tmp, tiles, ccells, bbox_part;
+  DevBuf offs, bboxes, status, grids, keys, vals, counts, cell_start, spts, tmp, tiles, ccells,
+      bbox_part;
   uint64_t n = 0;
   uint32_t nclouds = 0, ntiles = 0;
   uint64_t cap_cells = 0;
@@ -2602,7 +2664,7 @@ struct rtnn_graph_s {
   ~rtnn_graph_s() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
-    DevBuf* all[] = {&offs, &bboxes, &status, &grids, &keys, &vals, &cell_start, &spts, &tmp,
+    DevBuf* all[] = {&offs, &bboxes, &status, &grids, &keys, &vals, &counts, &cell_start, &spts, &tmp,
                      &tiles, &ccells, &bbox_part};
     for (DevBuf* b : all) b->release();
   }
@@ -2655,16 +2717,26 @@ hipError_t enqueue_batched(rtnn_graph g, const float* xyz, float cell, int mode,
   if ((e = plan_batched(g->bboxes.as<float>(), off, g->nclouds, cell, cells, g->cap_cells,
                         g->grids.as<GridDesc>(), status, st)) != hipSuccess)
     return e;
-  if ((e = cell_keys(xyz, g->n, g->grids.as<GridDesc>(), off, g->nclouds, keys, vals, nullptr,
-                     st)) != hipSuccess)
-    return e;
-  if ((e = radix_sort_pairs(keys, vals, g->n, bits_for(g->cap_cells - 1), g->tmp.as<uint32_t>(),
-                            st, nullptr)) != hipSuccess)
-    return e;
-  if ((e = cell_bounds(keys, g->n, (uint32_t)g->cap_cells, g->cell_start.as<uint32_t>(),
-                       g->tmp.as<uint32_t>(), st)) != hipSuccess)
-    return e;
-  if ((e = gather_points(xyz, vals, g->n, g->spts.as<float4>(), st)) != hipSuccess) return e;
+  if (count_cells_rule(g->n, g->cap_cells)) {
+    if ((e = cell_count(xyz, g->n, g->grids.as<GridDesc>(), off, g->nclouds,
+                        g->counts.as<uint32_t>(), keys, vals, st)) != hipSuccess)
+      return e;
+    if ((e = cell_scan_place(xyz, g->n, g->cap_cells, g->counts.as<uint32_t>(), keys, vals,
+                             g->cell_start.as<uint32_t>(), g->tmp.as<uint32_t>(),
+                             g->spts.as<float4>(), st)) != hipSuccess)
+      return e;
+  } else {
+    if ((e = cell_keys(xyz, g->n, g->grids.as<GridDesc>(), off, g->nclouds, keys, vals, nullptr,
+                       st)) != hipSuccess)
+      return e;
+    if ((e = radix_sort_pairs(keys, vals, g->n, bits_for(g->cap_cells - 1),
+                              g->tmp.as<uint32_t>(), st, nullptr)) != hipSuccess)
+      return e;
+    if ((e = cell_bounds(keys, g->n, (uint32_t)g->cap_cells, g->cell_start.as<uint32_t>(),
+                         g->tmp.as<uint32_t>(), st)) != hipSuccess)
+      return e;
+    if ((e = gather_points(xyz, vals, g->n, g->spts.as<float4>(), st)) != hipSuccess) return e;
+  }
   SearchArgs a;
   std::memset(&a, 0, sizeof a);
   a.spts = g->spts.as<float4>();
@@ -2729,7 +2801,14 @@ int rtnn_graph_batched(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets,
   CK(g->vals.ensure(4 * n));
   CK(g->cell_start.ensure(4 * (g->cap_cells + 1)));
   CK(g->spts.ensure(16 * n + kSptsPadBytes));
-  CK(g->tmp.ensure(4 * std::max(radix_tmp_words(n), cell_bounds_tmp_words(g->cap_cells))));
+  if (count_cells_rule(n, g->cap_cells)) {
+    CK(g->tmp.ensure(4 * cell_scan_tmp_words(g->cap_cells)));
+    // zero once; every run leaves them zero
+    CK(g->counts.ensure(4 * ((g->cap_cells + 3) & ~3ull)));
+    CK(fill_u32(g->counts.as<uint32_t>(), g->cap_cells, 0, ctx->st));
+  } else {
+    CK(g->tmp.ensure(4 * std::max(radix_tmp_words(n), cell_bounds_tmp_words(g->cap_cells))));
+  }
   CK(g->tiles.ensure(sizeof(Tile) * g->ntiles));
   CK(g->ccells.ensure(4 * (uint64_t)nclouds));
   if (nclouds == 1) CK(g->bbox_part.ensure(4 * 6 * kBboxBlocks));

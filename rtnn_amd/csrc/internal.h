@@ -46,6 +46,22 @@ hipError_t cell_keys_single(const float* xyz, uint64_t n, const GridDesc& g, Gri
 uint64_t cell_bounds_tmp_words(uint64_t ncells);
 hipError_t cell_bounds(const uint32_t* sorted_keys, uint64_t n, uint32_t ncells,
                        uint32_t* cell_start, uint32_t* tmp, hipStream_t st, int shift = 0);
+// Raster grid by counting, in two steps: keys[i] = cell of point i, ranks[i] =
+// its rank in the cell, counts[cell] += 1 (one cloud with its descriptor by
+// value, stored to *gstore, or clouds with theirs on the device); then
+// cell_start[0 .. ncells] and spts (a cell's points contiguous, in no
+// particular order).  counts (ncells words, 16-byte aligned) is zero before
+// the first step and again after the second.  tmp:
+// cell_scan_tmp_words(ncells) words.
+hipError_t cell_count_single(const float* xyz, uint64_t n, const GridDesc& g, GridDesc* gstore,
+                             uint32_t* counts, uint32_t* keys, uint32_t* ranks, hipStream_t st);
+hipError_t cell_count(const float* xyz, uint64_t n, const GridDesc* grids,
+                      const uint64_t* offsets, uint32_t nclouds, uint32_t* counts, uint32_t* keys,
+                      uint32_t* ranks, hipStream_t st);
+uint64_t cell_scan_tmp_words(uint64_t ncells);
+hipError_t cell_scan_place(const float* xyz, uint64_t n, uint64_t ncells, uint32_t* counts,
+                           const uint32_t* keys, const uint32_t* ranks, uint32_t* cell_start,
+                           uint32_t* tmp, float4* spts, hipStream_t st);
 // keys[i] = Morton code of point i's cell on the cubic level-0 grid g0.
 hipError_t morton_keys(const float* xyz, uint64_t n, const GridDesc* g0, uint32_t* keys,
                        uint32_t* vals, hipStream_t st);
