@@ -93,11 +93,9 @@ def workload(name):
                     # bucket, timed on 3M of the queries (about 0.1 s each)
                     proposal_tune={"sample": 3_000_000, "margins": [1.0, 1.5, 2.0, 3.0],
                                    "buckets": [0.0, 0.8]},
-                    # the octree walk of a 6-level hierarchical grid (fixed
-                    # configuration, not tuned): leaves of up to 65536
-                    # points, scanned chunk by chunk, two lanes per query
-                    options={"grid_levels": 6, "queries_per_wave": 0, "tree_leaf": 65536,
-                             "tree_lanes": 2},
+                    # the packet walk (fixed configuration, not tuned): one
+                    # lane per query on a hierarchical grid
+                    options={"grid_levels": 6, "queries_per_wave": 0},
                     cfg={"workload": "KNN K=32 r=100: 30M Levy-flight points (Pareto alpha 1.5, "
                                      "min step 0.01, periodic [0,1000]^3), 30M uniform queries",
                          "points": 30_000_000, "queries": 30_000_000, "k": 32, "radius": 100.0})
@@ -245,12 +243,13 @@ def proposal_tune(ctx, dq, r, k, spec, base_opts):
             "seconds": round(time.perf_counter() - t0, 3)}
 
 
-def kernel_name(res, mode, opts):
+def kernel_name(res, mode, opts, method):
     """Name of the dominant search kernel of a method's configuration."""
     o = opts or {}
     if res.get("lanes_per_query") == 1 and not o.get("group_buffer") == 3:
-        if mode == "knn" and o.get("grid_levels", 0) >= 2:
-            return "k_topk_treeg" if o.get("tree_lanes", 0) in (2, 4, 8) else "k_topk_tree"
+        if mode == "knn" and (method == "plain" or o.get("grid_levels", 0) >= 2 or
+                              (method == "partitioned" and not o.get("grid_levels"))):
+            return "k_knn_packet"
         return "k_topk_thread"
     if o.get("group_buffer") == 3:
         return "k_topk_pool"
@@ -454,7 +453,7 @@ def measure(args, wname, torch, rtnn_amd, extra=False):
         algo = c27_bytes(pts, pts if qs is None else qs, r, k)
         algo_def = "range bytes per query 12 + 12*C27(q) + 4*K"
     achieved = algo / (kms * 1e-3) / 1e9
-    kname = kernel_name(results[kroof], mode, opts_used.get(kroof))
+    kname = kernel_name(results[kroof], mode, opts_used.get(kroof), kroof)
     pmc = pmc_row(wname, kname)
     roof = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 5),

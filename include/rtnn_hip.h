@@ -60,7 +60,10 @@ typedef struct {
   uint32_t max_cells;     /* cap on grid cells (cell edge grows to respect it)      */
   int   grid_levels;      /* learned/partitioned KNN: 1 = one raster grid of edge
                              r / cell_factor; >= 2 = hierarchical Morton grid with
-                             that many levels (edges r, r/2, ...); 0 = auto       */
+                             that many levels (edges r, r/2, ...), or with one lane
+                             per query (queries_per_wave 0 or 64, k <= 64) the
+                             packet walk over a box tree; 0 = auto (learned 1,
+                             partitioned 5)                                       */
   float level_alpha;      /* hierarchical: a query of radius R walks the finest
                              level whose cell edge is >= R * level_alpha (0: 1.0) */
   int   group_buffer;     /* group kernel's LDS hit buffer per query: 0 auto / 2
@@ -75,11 +78,9 @@ typedef struct {
                              wave stages the points of its queries' union block in
                              LDS (up to that many per wave) and scans them there
                              (1 = 512; 0 = off); implies compact buffers        */
-  int   tree_leaf;        /* hierarchical-grid KNN, one lane per query (the octree
-                             walk): a cell of at most this many points is scanned
-                             (chunk by chunk, 32 points per bounding box) instead
-                             of descended into; 0 = 256.  Large values suit very
-                             clustered points (Levy flights: 65536)            */
+  int   tree_leaf;        /* no effect any more (the leaves of the walk that one lane
+                             per query takes over a hierarchical grid are fixed);
+                             checked (>= 0) and kept for callers that set it     */
   float bucket_ratio;     /* learned/partitioned KNN, density buckets: a query whose
                              proposed radius r' >= bucket_ratio * r is searched at
                              r at once (its row is final after the first launch:
@@ -89,11 +90,9 @@ typedef struct {
                              first radius, which holds k neighbours), so queries
                              the partition bounds more tightly keep its radius
                              and do not fall back; 0 = the network alone        */
-  int   tree_lanes;       /* hierarchical-grid KNN, the octree walk: lanes per
-                             query (2, 4 or 8 split the chunks and points of
-                             every leaf; 0 or 1 = one lane).  2 is the fastest
-                             on clustered points (Levy flights)               */
-  int   tree_fallback;    /* hierarchical-grid KNN with the octree walk (k <= 64):
+  int   tree_lanes;       /* no effect any more (that walk takes one lane per
+                             query); checked (0, 1, 2, 4 or 8)                  */
+  int   tree_fallback;    /* hierarchical-grid KNN (k <= 64), the packet walk:
                              0 = the rows short at their proposed radius are
                              searched once more at r; 1 = through the radius-
                              growth stages (as on raster grids)               */
@@ -182,7 +181,10 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
  * points gives a launch radius min(r, sqrt(3)*(iter+1)*cell); a query whose
  * sphere holds fewer than k hits is searched again at a grown radius (up to
  * four growth stages, then r; a row searched at r is final), so the result
- * equals rtnn_search(..., RTNN_MODE_KNN, ...). */
+ * equals rtnn_search(..., RTNN_MODE_KNN, ...).  With one lane per query on a
+ * hierarchical grid (the default) the packet walk takes the place of the launch
+ * radius: every query is searched at r, bounded from its first leaves on by the
+ * k-th nearest point found so far, so no row is short. */
 int rtnn_search_partitioned(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
                             float r, uint32_t k,
                             int32_t* out_idx, float* out_d2, int out_on_device,

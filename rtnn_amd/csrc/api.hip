@@ -210,7 +210,6 @@ struct rtnn_ctx_s {
   // grid
   DevBuf keys, vals, counts, cell_start, spts, tmp, grids;
   uint64_t counts_zero = 0;  // leading words of `counts` known to be zero
-  DevBuf cboxes;  // hierarchical grids: bounding box per kChunkPts sorted points
   DevBuf boxes;   // box tree of the packet walk
   GridDesc hgrid{};
   uint64_t ncells = 0;
@@ -266,7 +265,7 @@ struct rtnn_ctx_s {
     DevBuf* all[] = {&pts, &keys, &vals, &counts, &cell_start, &spts, &tmp, &grids,
                      &qin, &qkeys, &qvals, &qsorted, &oidx, &od2, &shortrows, &misc,
                      &tiles, &offs, &bboxes, &pgrid, &pcounts, &qradius, &tr_q, &tr_idx,
-                     &tr_d2, &tr_t, &tr_f, &tr_out, &bcnt, &boff, &bpairs, &cboxes, &ovf,
+                     &tr_d2, &tr_t, &tr_f, &tr_out, &bcnt, &boff, &bpairs, &ovf,
                      &boxes};
     for (DevBuf* b : all) b->release();
     if (st3) (void)hipStreamSynchronize(st3);
@@ -535,10 +534,10 @@ int build_hgrid(rtnn_ctx ctx, float r, int want_levels) {
     CK(cell_bounds(ctx->keys.as<uint32_t>(), n, (uint32_t)(1ull << (3 * (b - l))),
                    ctx->cell_start.as<uint32_t>() + lv[l].cell_base, ctx->tmp.as<uint32_t>(),
                    ctx->st, 3 * l));
-  CK(gather_points(ctx->pts.as<float>(), ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(),
-                   ctx->st));
-  CK(ctx->cboxes.ensure(32 * ((n + kChunkPts - 1) / kChunkPts) + 32));
-  CK(chunk_boxes(ctx->spts.as<float4>(), n, ctx->cboxes.as<float4>(), ctx->st));
+  // The box tree of the packet walk, which searches the short rows.
+  CK(ctx->boxes.ensure(32 * box_tree_layout(n, nullptr).boxes));
+  CK(build_box_tree(ctx->pts.as<float>(), ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(),
+                    box_tree_layout(n, ctx->boxes.as<float4>()), ctx->st));
   ctx->ncells = total;
   ctx->spts_current = true;
   ctx->hlevels = L;
@@ -590,9 +589,10 @@ constexpr int kQueryKeyBits = 8;  // Morton bits per axis of the query order
 // Returns the processing-order array through *qproc.  The ordering runs on
 // ctx->st2, started by ctx->ev_desc (recorded by the grid build once its
 // descriptors are on the device), so it overlaps the point sort on ctx->st;
-// ctx->st waits for it before returning work that reads *qproc.
+// ctx->st waits for it before returning work that reads *qproc.  always_order:
+// the packet walk of the proposal methods, which needs neighbours in a wave.
 int prepare_queries(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
-                    const float4** qproc, int key_bits = kQueryKeyBits) {
+                    const float4** qproc, int key_bits = kQueryKeyBits, bool always_order = false) {
   if (!qxyz) {  // the points themselves, already in cell order
     *qproc = ctx->spts.as<float4>();
     return RTNN_OK;
@@ -609,7 +609,7 @@ int prepare_queries(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
     CK(hipMemcpyAsync(ctx->qin.p, qxyz, 12 * nq, hipMemcpyHostToDevice, s2));
     dq = ctx->qin.as<float>();
   }
-  if (ctx->opt.query_order == 1) {
+  if (ctx->opt.query_order == 1 && !always_order) {
     CK(iota_u32(ctx->qvals.as<uint32_t>(), nq, s2));
   } else {
     // Morton order of the query cells, 8 bits per axis (cells merged in
@@ -700,9 +700,6 @@ SearchArgs base_args(rtnn_ctx ctx, const float4* qproc, uint64_t nq, float r, ui
     a.nlevels = ctx->hlevels;
     a.level_min = ctx->hlevel_min;
     a.level_alpha = ctx->opt.level_alpha > 0 ? ctx->opt.level_alpha : 1.0f;
-    a.chunk_box = ctx->cboxes.as<float4>();
-    a.tree_leaf = ctx->opt.tree_leaf > 0 ? (uint32_t)ctx->opt.tree_leaf : kTreeLeafDefault;
-    a.tree_lanes = ctx->opt.tree_lanes > 1 ? (uint32_t)ctx->opt.tree_lanes : 1u;
   }
   return a;
 }
@@ -1144,9 +1141,14 @@ namespace {
 
 // Point-count grid over ctx->pts with edge `cell` (origin = points' bbox min).
 // grow = false: the edge is kept (error if the grid would exceed the budget).
-int build_count_grid(rtnn_ctx ctx, float cell, bool grow) {
+// wide: a grid of up to 1024 cells per axis is within the budget whatever its
+// cells (what the tables of the hierarchical grid hold).
+int build_count_grid(rtnn_ctx ctx, float cell, bool grow, bool wide = false) {
   GridDesc g;
-  const uint64_t cap = max_cells_for(ctx, ctx->n);
+  uint64_t cap = max_cells_for(ctx, ctx->n);
+  plan_grid(ctx->bbox, cell, g);
+  if (wide && std::max(g.dim[0], std::max(g.dim[1], g.dim[2])) <= 1024)
+    cap = std::max<uint64_t>(cap, 1ull << 30);
   for (int tries = 0;; ++tries) {
     plan_grid(ctx->bbox, cell, g);
     if (grid_cells(g) <= cap && grid_cells(g) < 0xfffffff0ull) break;
@@ -1194,12 +1196,15 @@ int partition_proposals(rtnn_ctx ctx, bool hier, const float4* qproc, uint64_t n
   return RTNN_OK;
 }
 
+int proposal_levels(rtnn_ctx ctx, Proposal kind) {
+  return ctx->opt.grid_levels > 0 ? ctx->opt.grid_levels : (kind == Proposal::kLearned ? 1 : 5);
+}
+
 int compute_proposals(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq, int on_device,
                       float r, uint32_t k, const float4** qproc_out) {
   const float f = ctx->opt.cell_factor > 0 ? ctx->opt.cell_factor
                                            : (kind == Proposal::kLearned ? 2.0f : 4.0f);
-  const int levels = ctx->opt.grid_levels > 0 ? ctx->opt.grid_levels
-                                              : (kind == Proposal::kLearned ? 1 : 5);
+  const int levels = proposal_levels(ctx, kind);
   bool hier = levels >= 2;
   int rc = hier ? build_hgrid(ctx, r, levels) : build_grid(ctx, r / f);
   if (rc == RTNN_ERR_UNSUPPORTED && hier) {
@@ -1251,6 +1256,32 @@ int compute_proposals(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t n
   return RTNN_OK;
 }
 
+// The proposals of a search that walks packets: the box tree and the queries in
+// its order; the MLP's radii from the counts of the edge-r cells (the cells of
+// the hierarchical grid's top level).  The density partition needs no radii
+// here: they would bound a query's sphere by a cube that holds k points, and the
+// walk, which starts from the leaves around the query, is bounded by the k-th
+// point found so far.  Its rows are searched at r and none falls short (Gaussian
+// mixture, 1M, K = 8: radii and their level tables took 0.45 ms of a pass).
+int packet_proposals(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq, int on_device,
+                     float r, const float4** qproc, BoxTree* tree) {
+  int rc = build_packet_tree(ctx, tree);
+  if (rc) return rc;
+  rc = prepare_queries(ctx, qxyz, nq, on_device, qproc, kPacketKeyBits, true);
+  if (rc) return rc;
+  CK(hipEventRecord(ctx->ev[1], ctx->st));
+  CK(ctx->qradius.ensure(4 * nq));
+  if (kind != Proposal::kLearned) return RTNN_OK;
+  rc = build_count_grid(ctx, r, false, true);
+  if (rc) return rc;
+  CK(mlp_propose(ctx->mlp, *qproc, (uint32_t)nq, ctx->pgrid.as<GridDesc>(), false,
+                 ctx->pcounts.as<uint32_t>(), r, false, ctx->qradius.as<float>(), ctx->st,
+                 ctx->num_cus));
+  if (ctx->opt.bucket_ratio > 0.0f)
+    CK(bucket_snap(ctx->qradius.as<float>(), (uint32_t)nq, ctx->opt.bucket_ratio * r, r, ctx->st));
+  return RTNN_OK;
+}
+
 // KNN with a proposed radius r' <= r per query, then an exact fallback: the
 // rows with fewer than k hits within r' are searched again at r.  If a row
 // has >= k hits with d2 < r'^2 <= r^2, any other point has d2 >= r'^2, so
@@ -1273,8 +1304,19 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
   CK(hipSetDevice(ctx->device));
   CK(hipEventRecord(ctx->ev[0], ctx->st));
   const float4* qproc = nullptr;
-  rc = compute_proposals(ctx, kind, qxyz, nq, on_device, r, k, &qproc);
+  // One query per lane on a hierarchical grid: the packet walk over the box
+  // tree, which needs no level tables (learned_cap does: it takes the
+  // partition's radii from them).
+  const int gl = group_lanes_from_opt(ctx, RTNN_MODE_KNN, k);
+  BoxTree tree{};
+  const bool packet = proposal_levels(ctx, kind) >= 2 && gl == 1 && k <= 64 &&
+                      !pool_requested(ctx, k) &&
+                      !(kind == Proposal::kLearned && ctx->opt.learned_cap != 0);
+  rc = packet ? packet_proposals(ctx, kind, qxyz, nq, on_device, r, &qproc, &tree)
+              : compute_proposals(ctx, kind, qxyz, nq, on_device, r, k, &qproc);
   if (rc) return rc;
+  if (ctx->hlevels > 0) tree = box_tree_layout(ctx->n, ctx->boxes.as<float4>());
+  const bool walk = packet || ctx->hlevels > 0;  // `tree` stands over spts
   CK(hipEventRecord(ctx->ev[2], ctx->st));
   OutBufs o;
   rc = output_targets(ctx, nq, k, out_idx, out_d2, out_on_device, o);
@@ -1286,13 +1328,12 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
   uint32_t* hits[2] = {lists[0] + 2 * nq, lists[0] + 3 * nq};
   uint32_t* counters = lists[0] + 4 * nq;
   CK(fill_u32(counters, kGrowStages + 1, 0, ctx->st));
-  const int gl = group_lanes_from_opt(ctx, RTNN_MODE_KNN, k);
   const bool pooled = pool_requested(ctx, k) && ctx->hlevels == 0;
   if (!pooled && (gl < 0 || k > max_k_for_group(gl)))
     return fail(ctx, RTNN_ERR_UNSUPPORTED, "k=%u not supported by the selected kernel", k);
   // Stage 1: every query at its proposed radius r'.
   SearchArgs a = base_args(ctx, qproc, nq, r, k, o);
-  a.qradius = ctx->qradius.as<float>();
+  a.qradius = packet && kind == Proposal::kPartition ? nullptr : ctx->qradius.as<float>();
   a.short_rows = lists[0];
   a.short_count = &counters[0];
   a.short_hits = hits[0];
@@ -1300,8 +1341,11 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
     rc = arm_overflow(ctx, nq, a);
     if (rc) return rc;
   }
-  CK(launch_search(a, 1, gl, ctx->st, ctx->num_cus, wide_buffers(ctx), tile_points(ctx), false,
-                   pooled ? ctx->opt.queries_per_wave : 0));
+  if (walk && gl == 1)
+    CK(launch_knn_packet(a, tree, ctx->st, ctx->num_cus));
+  else
+    CK(launch_search(a, 1, gl, ctx->st, ctx->num_cus, wide_buffers(ctx), tile_points(ctx), false,
+                     pooled ? ctx->opt.queries_per_wave : 0));
   CK(hipEventRecord(ctx->ev[3], ctx->st));
   // Growth stages: a row short at radius R (m < k hits) is searched again at
   // min(r, R * hit_scale(m, k)), hit_scale in [1.15, 2]; the radius it used is
@@ -1311,14 +1355,11 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
   // query with wide, deep buffers (k <= 64 here; room for 2 max(k, 32) keys)
   // measured faster than one lane (C3: 1.25 -> 0.84 ms), two lanes, or the
   // k <= 16 buffer.
-  // The octree walk (hierarchical grid, one lane per query) costs about as
-  // much at a grown radius as at r -- its limit, not its radius, bounds the
-  // walk -- so its short rows go straight to the last stage: on the
-  // Levy-flight KNN 151 short rows took 27 ms through five stages, since
-  // each stage waits for its slowest walk.  Where many rows fall back at
-  // radii well below r the stages can still pay (option tree_fallback = 1,
-  // which the autotuner tries).
-  const bool tree_fallback = ctx->hlevels > 0 && k <= 64 && ctx->opt.tree_fallback == 0;
+  // The packet walk costs about as much at a grown radius as at r -- its limit,
+  // not its radius, bounds it -- so its short rows go straight to the last
+  // stage (option tree_fallback = 1: through the growth stages, which the
+  // autotuner tries).
+  const bool tree_fallback = walk && k <= 64 && ctx->opt.tree_fallback == 0;
   for (int j = tree_fallback ? kGrowStages : 0; j <= kGrowStages; ++j) {
     SearchArgs s = base_args(ctx, qproc, nq, r, k, o);
     s.qsel = tree_fallback ? lists[0] : lists[j & 1];
@@ -1331,11 +1372,13 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
       s.short_hits = hits[(j + 1) & 1];
       s.short_count = &counters[j + 1];
     }
-    // On the hierarchical grid the octree walk (one lane per query) prunes
-    // by its shrinking limit, which pays most for these wide searches.
     // Beyond k = 64 (the register top-k and the 4-lane buffers) the rows go
     // to 16- or 64-lane groups.
-    const int fl = k > 256 ? 64 : k > 64 ? 16 : ctx->hlevels > 0 ? 1 : kFallbackLanes;
+    if (walk && k <= 64) {
+      CK(launch_knn_packet(s, tree, ctx->st, ctx->num_cus));
+      continue;
+    }
+    const int fl = k > 256 ? 64 : k > 64 ? 16 : kFallbackLanes;
     CK(launch_search(s, 1, fl, ctx->st, ctx->num_cus, true, false, true));
   }
   CK(hipEventRecord(ctx->ev[4], ctx->st));
@@ -2313,35 +2356,33 @@ int rtnn_autotune(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device, i
     float cf;
     int qpw, levels;
     float alpha;
-    int buffer, tile, leaf;
-    int tlanes = 0;
+    int buffer, tile;
   };
   std::vector<Cand> cands;
   for (int i = 0; i < ncf; ++i)
     for (int j = 0; j < nqpw; ++j) {
       const bool group = qpws[j] > 0 && qpws[j] < 64;
-      cands.push_back({cfs[i], qpws[j], plain ? 0 : 1, 0.0f, group ? 2 : 0, 0, 0});
+      if (plain && !range && !group && i > 0) continue;  // the packet walk has no cells
+      cands.push_back({cfs[i], qpws[j], plain ? 0 : 1, 0.0f, group ? 2 : 0, 0});
       if (group) {
-        cands.push_back({cfs[i], qpws[j], plain ? 0 : 1, 0.0f, 1, 0, 0});
+        cands.push_back({cfs[i], qpws[j], plain ? 0 : 1, 0.0f, 1, 0});
         if (qpws[j] != 32)  // 2-lane groups have no tiled kernel
           for (int tp : {256, 512, 1024})
-            cands.push_back({cfs[i], qpws[j], plain ? 0 : 1, 0.0f, 1, tp, 0});
+            cands.push_back({cfs[i], qpws[j], plain ? 0 : 1, 0.0f, 1, tp});
       }
     }
   // The pooled kernel (k <= 64): 16, 32 or 64 queries per wave share one
   // candidate pool (raster grids).
   if (k <= 64)
     for (int i = 0; i < ncf; ++i)
-      for (int qpw : {16, 32, 64}) cands.push_back({cfs[i], qpw, plain ? 0 : 1, 0.0f, 3, 0, 0});
-  // Hierarchical grids: the octree walk (one lane per query) with leaves of
-  // 256 or 65536 points, and 4-lane groups on the level rule.
-  if (!plain)
+      for (int qpw : {16, 32, 64}) cands.push_back({cfs[i], qpw, plain ? 0 : 1, 0.0f, 3, 0});
+  // Hierarchical grids: the packet walk (one lane per query), which does not
+  // depend on the levels, and 4-lane groups on the level rule.
+  if (!plain) {
+    cands.push_back({0.0f, 0, 5, 0.0f, 0, 0});
     for (int lv : {3, 5})
-      for (float al : {1.0f, 0.5f}) {
-        for (int leaf : {0, 65536})
-          for (int tl : {1, 2}) cands.push_back({0.0f, 0, lv, al, 0, 0, leaf, tl});
-        cands.push_back({0.0f, 16, lv, al, 0, 0, 0});
-      }
+      for (float al : {1.0f, 0.5f}) cands.push_back({0.0f, 16, lv, al, 0, 0});
+  }
   for (const Cand& cand : cands) {
     {
       const int qpw = cand.qpw;
@@ -2354,8 +2395,6 @@ int rtnn_autotune(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device, i
       ctx->opt.level_alpha = cand.alpha;
       ctx->opt.group_buffer = cand.buffer;
       ctx->opt.lds_tile = cand.tile;
-      ctx->opt.tree_leaf = cand.leaf;
-      ctx->opt.tree_lanes = cand.tlanes;
       double ms = 0.0;
       const int rc = time_candidate(
           [&](rtnn_stats* st) {
@@ -2376,9 +2415,9 @@ int rtnn_autotune(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device, i
         return rc;
       }
       tune_log("autotune %s: candidate %zu/%zu cell_factor %g qpw %d levels %d alpha %g "
-               "buffer %d tile %d leaf %d tree lanes %d: %.4f ms", method_name(method),
+               "buffer %d tile %d: %.4f ms", method_name(method),
                (size_t)(&cand - cands.data()) + 1, cands.size(), cand.cf, cand.qpw, cand.levels,
-               cand.alpha, cand.buffer, cand.tile, cand.leaf, cand.tlanes, ms);
+               cand.alpha, cand.buffer, cand.tile, ms);
       if (ms < best_t) {
         best_t = ms;
         best_opt = ctx->opt;
@@ -2464,7 +2503,7 @@ int rtnn_autotune(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device, i
       ctx->opt = best_opt;
     }
     if (best_opt.grid_levels >= 2 && best_opt.queries_per_wave == 0 && k <= 64) {
-      // The octree walk's short rows: at r at once, or through the growth stages.
+      // The packet walk's short rows: at r at once, or through the growth stages.
       ctx->opt.tree_fallback = 1 - best_opt.tree_fallback;
       double ms = 0.0;
       const int rc = time_candidate(

@@ -77,12 +77,6 @@ struct SearchArgs {
   int nlevels;
   int level_min;
   float level_alpha;
-  // nullable: bounding box of every kChunkPts consecutive sorted points
-  // (chunk c: min at [2c], max at [2c+1]); the octree walk skips the chunks of
-  // a large leaf that lie beyond its limit.
-  const float4* chunk_box;
-  uint32_t tree_leaf;  // octree walk: cells of at most this many points are leaves
-  uint32_t tree_lanes;  // octree walk: lanes per query (1: k_topk_tree; 2, 4, 8: k_topk_treeg)
   // Pooled kernel (k_topk_pool): a query with more hits than its LDS buffer
   // holds appends its processing position here (count in ovf_count); the
   // group kernel then searches those rows again.
@@ -104,10 +98,6 @@ struct BoxTree {
   int top;
   uint64_t boxes;  // of all levels
 };
-
-constexpr uint32_t kTreeLeafDefault = 256;
-
-constexpr uint32_t kChunkPts = 32;
 
 constexpr int kTileQ = 256;  // queries per tile (= threads of a KNN block)
 

@@ -71,8 +71,6 @@ hipError_t count_sorted(const float4* spts, uint64_t n, const GridDesc* g, uint3
 // spts[j] = (xyz[vals[j]], bits(vals[j])).
 hipError_t gather_points(const float* xyz, const uint32_t* vals, uint64_t n, float4* spts,
                          hipStream_t st);
-// Bounding box of every kChunkPts consecutive points of spts (2 float4 each).
-hipError_t chunk_boxes(const float4* spts, uint64_t n, float4* box, hipStream_t st);
 // Morton key (10 bits per axis) of each query's cell in grid g, shifted right
 // by `shift` bits per axis (shift < 0: derived on the device from g's widest
 // axis, keeping 8 bits per axis); vals[i] = i.

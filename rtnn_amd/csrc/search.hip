@@ -97,14 +97,14 @@ __device__ inline void topk_insert(uint64_t (&list)[KC], uint64_t key) {
   list[0] = list[0] > key ? key : list[0];
 }
 
-// Waves per SIMD asked of the compiler (as for the octree walks: a latency-
-// bound walk, residency before registers).  Spheres KNN, K = 16 (10M x 10M,
+// Waves per SIMD asked of the compiler (a latency-bound walk: residency before
+// registers).  Spheres KNN, K = 16 (10M x 10M,
 // r = 10): 10.07 ms at 117 VGPRs (four waves), 8.60 ms at 90 (five, no
 // spills); Gaussian-mixture KNN, K = 8: 10.01 / 10.00 ms.
 template <int KC>
 constexpr int thread_waves() { return KC <= 8 ? 8 : KC <= 16 ? 5 : KC <= 32 ? 3 : 1; }
 
-template <int KC, bool KNN, bool HIER>
+template <int KC, bool KNN>
 __global__ __launch_bounds__(kTileQ) __attribute__((amdgpu_waves_per_eu(thread_waves<KC>())))
 void k_topk_thread(const SearchArgs a) {
   const uint32_t nq = launch_nq(a);
@@ -123,44 +123,20 @@ void k_topk_thread(const SearchArgs a) {
     cell_range(g, qv.x, R, 0, lo0, hi0);
     cell_range(g, qv.y, R, 1, lo1, hi1);
     cell_range(g, qv.z, R, 2, lo2, hi2);
-    uint32_t lvl_base = g.cell_base;
-    if (HIER) {
-      // Finest built level whose cell is >= R * alpha; the level-0 range
-      // shifted right by the level is that level's range (floor division is
-      // monotone and keeps empty ranges empty).
-      int lvl = a.level_min;
-      float c = ldexpf(g.cell, lvl);
-      const float want = R * a.level_alpha;
-      while (lvl < a.nlevels - 1 && c < want) {
-        c *= 2.0f;
-        ++lvl;
-      }
-      lo0 >>= lvl; hi0 >>= lvl; lo1 >>= lvl; hi1 >>= lvl; lo2 >>= lvl; hi2 >>= lvl;
-      lvl_base = a.grids[lvl].cell_base;
-    }
     const int nx = hi0 - lo0 + 1, ny = hi1 - lo1 + 1, nz = hi2 - lo2 + 1;
-    // raster: one run per (y, z) row; hierarchical: one run per Morton cell
-    const int nrows = (active && nx > 0 && ny > 0 && nz > 0) ? (HIER ? nx : 1) * ny * nz : 0;
+    const int nrows = (active && nx > 0 && ny > 0 && nz > 0) ? ny * nz : 0;  // (y, z) rows
 
     uint64_t list[KC];
 #pragma unroll
     for (int i = 0; i < KC; ++i) list[i] = ~0ull;
 
-    // One contiguous run of sorted points per raster row (or Morton cell).
+    // One contiguous run of sorted points per row.
     auto row_bounds = [&](int rr, uint32_t& s, uint32_t& e) {
-      if (HIER) {
-        const int cx = lo0 + rr % nx, t = rr / nx;
-        const int cy = lo1 + t % ny, cz = lo2 + t / ny;
-        const uint32_t id = lvl_base + morton3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
-        s = a.cell_start[id];
-        e = a.cell_start[id + 1];
-      } else {
-        const int cy = lo1 + rr % ny, cz = lo2 + rr / ny;
-        const uint32_t rowc = lvl_base + ((uint32_t)cz * (uint32_t)g.dim[1] + (uint32_t)cy) *
-                                             (uint32_t)g.dim[0];
-        s = a.cell_start[rowc + lo0];
-        e = a.cell_start[rowc + hi0 + 1];
-      }
+      const int cy = lo1 + rr % ny, cz = lo2 + rr / ny;
+      const uint32_t rowc = g.cell_base + ((uint32_t)cz * (uint32_t)g.dim[1] + (uint32_t)cy) *
+                                              (uint32_t)g.dim[0];
+      s = a.cell_start[rowc + lo0];
+      e = a.cell_start[rowc + hi0 + 1];
     };
     // The next run's bounds are loaded while the current run is scanned.
     uint32_t s_next = 0, e_next = 0;
@@ -207,380 +183,6 @@ void k_topk_thread(const SearchArgs a) {
       for (int i = 0; i < KC; ++i) hits += ((uint32_t)i < k && list[i] != ~0ull) ? 1u : 0u;
       append_short(a, hits < k && R < a.r, qs, hits, R);  // a row searched at r is final
     }
-  }
-}
-
-// --------------------------------------------------------------------------
-// KNN on the hierarchical Morton grid: octree walk, one query per lane
-//
-// A level-l cell m has children 8m .. 8m+7 at level l-1 (the Morton key
-// nests), and every cell's points are one contiguous run of the sorted
-// points, so the levels form an implicit octree.  From each top-level cell
-// within [q - R, q + R] the walk goes depth first, the child holding the
-// query first (child j visits octant j ^ the query's octant), without a
-// stack: the position among siblings is recovered from the key.  A cell
-// whose padded box lies farther than the current limit is skipped; a cell of
-// the finest built level, or holding at most a.tree_leaf points, is scanned,
-// chunk by chunk: the bounding box of every kChunkPts sorted points skips the
-// chunks beyond the limit.  The leaf size is an option: on the full-size
-// Levy-flight KNN (learned radius) a step took 6.9 s with leaves of up to 256
-// points, 4.1 s with 4096, 1.3 s with 65536; the Gaussian-mixture KNN (1M
-// points) is fastest at 256 (2.9 ms, 3.5 ms with 65536).
-// Top-level cells are taken in rings of growing distance around the query's
-// own, so the limit shrinks early.
-// The limit starts at the float below R^2 and, once k keys are held, drops
-// to the k-th key's d2, so a dense cluster beyond the k nearest is cut off
-// at its coarsest cell.  The result is the same as the cube walk's: only
-// cells that cannot hold a hit (d2 <= limit) are skipped.
-
-__device__ inline uint32_t compact3(uint32_t x) {
-  x &= 0x09249249u;
-  x = (x | (x >> 2)) & 0x030c30c3u;
-  x = (x | (x >> 4)) & 0x0300f00fu;
-  x = (x | (x >> 8)) & 0xff0000ffu;
-  x = (x | (x >> 16)) & 0x000003ffu;
-  return x;
-}
-
-// Squared distance from q to cell (ix, iy, iz) of edge c, the box grown by
-// pad on every side (a lower bound for any point the FP32 cell mapping puts
-// in the cell).
-__device__ inline float box_d2(const float4& q, const GridDesc& g0, float c, float pad,
-                               uint32_t ix, uint32_t iy, uint32_t iz) {
-  const float lx = g0.mn[0] + (float)ix * c - pad, hx = lx + c + 2.0f * pad;
-  const float ly = g0.mn[1] + (float)iy * c - pad, hy = ly + c + 2.0f * pad;
-  const float lz = g0.mn[2] + (float)iz * c - pad, hz = lz + c + 2.0f * pad;
-  const float dx = fmaxf(fmaxf(lx - q.x, q.x - hx), 0.0f);
-  const float dy = fmaxf(fmaxf(ly - q.y, q.y - hy), 0.0f);
-  const float dz = fmaxf(fmaxf(lz - q.z, q.z - hz), 0.0f);
-  return dx * dx + dy * dy + dz * dz;
-}
-
-// Waves per SIMD asked of the compiler for the octree walks: the walk is
-// bound by the latency of its dependent loads, so residency pays more than
-// registers, up to a few spilled ones.  Levy-flight KNN (30M points, 30M
-// uniform queries, r = 100), K = 32, two lanes: 908 ms at 137 VGPRs (three
-// waves per SIMD), 756 ms at 128 (four; 48 bytes spilled), 726 ms at 96
-// (five; 176 bytes); one lane: 1094 ms at 193 VGPRs (two waves), 802 ms at
-// 168 (three), 993 ms at 128 (four; 264 bytes).  K = 16, two lanes: 473 ms
-// at 105 VGPRs (four waves), 411 at 96 (five), 379 at 80 (six); one lane:
-// 544 ms at 154 (three), 381 at 95 (five), 351 at 80 (six).  K = 8, two
-// lanes: 328 ms at 88 (five), 302 at 80 (six), 283 at 64 (eight); one lane:
-// 363 ms at 106 (four), 307 at 80 (six), 295 at 64 (eight).  Six waves at
-// K = 32 spill 248 bytes and take 1402 ms.  Rows are unchanged throughout.
-// Beyond K = 32 no target is set (1: the compiler's own choice).
-template <int KC>
-constexpr int treeg_waves() { return KC <= 8 ? 8 : KC <= 16 ? 6 : KC <= 32 ? 5 : 1; }
-template <int KC>
-constexpr int tree_waves() { return KC <= 8 ? 8 : KC <= 16 ? 6 : KC <= 32 ? 3 : 1; }
-
-template <int KC>
-__global__ __launch_bounds__(kTileQ) __attribute__((amdgpu_waves_per_eu(tree_waves<KC>())))
-void k_topk_tree(const SearchArgs a) {
-  __shared__ uint32_t s_base[8];
-  if (threadIdx.x < 8) s_base[threadIdx.x] = (int)threadIdx.x < a.nlevels ?
-                                               a.grids[threadIdx.x].cell_base : 0u;
-  __syncthreads();
-  const uint32_t nq = launch_nq(a);
-  const int T = a.nlevels - 1, L0 = a.level_min;
-  const GridDesc g0 = a.grids[0];
-  for (TileIter it(a, nq); it.t < it.end; it.t += it.step) {
-    uint32_t q0, q1, gi;
-    tile_of(a, nq, it.t, q0, q1, gi);
-    const uint32_t qi = q0 + threadIdx.x;
-    if (qi >= q1) continue;
-    const uint32_t qs = a.qsel ? a.qsel[qi] : qi;
-    const float4 qv = a.queries[qs];
-    const uint32_t row = __float_as_uint(qv.w);
-    const float R = query_radius(a, qi, qs);
-    float lim = r2_limit(R * R);
-    uint64_t list[KC];
-#pragma unroll
-    for (int i = 0; i < KC; ++i) list[i] = ~0ull;
-    // top-level cells of [q - R, q + R] (the level-0 range shifted by T)
-    int lo0, hi0, lo1, hi1, lo2, hi2;
-    cell_range(g0, qv.x, R, 0, lo0, hi0);
-    cell_range(g0, qv.y, R, 1, lo1, hi1);
-    cell_range(g0, qv.z, R, 2, lo2, hi2);
-    // the query's level-0 cell (clamped): its octant at every level
-    const int qc0 = min(max((int)floorf((qv.x - g0.mn[0]) * g0.inv), 0), g0.dim[0] - 1);
-    const int qc1 = min(max((int)floorf((qv.y - g0.mn[1]) * g0.inv), 0), g0.dim[1] - 1);
-    const int qc2 = min(max((int)floorf((qv.z - g0.mn[2]) * g0.inv), 0), g0.dim[2] - 1);
-    const uint32_t qm = morton3((uint32_t)qc0, (uint32_t)qc1, (uint32_t)qc2);
-    const float mag = fabsf(g0.mn[0]) + fabsf(g0.mn[1]) + fabsf(g0.mn[2]) + fabsf(qv.x) +
-                      fabsf(qv.y) + fabsf(qv.z) + (float)g0.dim[0] * g0.cell;
-    if (hi0 >= lo0 && hi1 >= lo1 && hi2 >= lo2) {
-      const int tl0 = lo0 >> T, th0 = hi0 >> T, tl1 = lo1 >> T, th1 = hi1 >> T;
-      const int tl2 = lo2 >> T, th2 = hi2 >> T;
-      // Top-level cells in rings of growing Chebyshev distance around the
-      // query's own top cell, so the nearest points come first and the
-      // limit shrinks before the far cells are tested (each cell of the
-      // range is on exactly one ring; the result does not depend on order).
-      const int qt0 = qc0 >> T, qt1 = qc1 >> T, qt2 = qc2 >> T;
-      const int nring = max(max(max(qt0 - tl0, th0 - qt0), max(qt1 - tl1, th1 - qt1)),
-                            max(qt2 - tl2, th2 - qt2));
-      for (int ring = 0; ring <= nring; ++ring)
-      for (int tz = max(tl2, qt2 - ring); tz <= min(th2, qt2 + ring); ++tz)
-        for (int ty = max(tl1, qt1 - ring); ty <= min(th1, qt1 + ring); ++ty)
-          for (int tx = max(tl0, qt0 - ring); tx <= min(th0, qt0 + ring); ++tx) {
-            if (max(max(abs(tx - qt0), abs(ty - qt1)), abs(tz - qt2)) != ring) continue;
-            int l = T;
-            uint32_t m = morton3((uint32_t)tx, (uint32_t)ty, (uint32_t)tz);
-            for (;;) {
-              const float c = ldexpf(g0.cell, l);
-              const float pad = c * 0x1.0p-12f + mag * 0x1.0p-19f;
-              const float bd = box_d2(qv, g0, c, pad, compact3(m), compact3(m >> 1),
-                                      compact3(m >> 2));
-              bool down = false;
-              if (bd <= lim * 1.001f) {
-                const uint32_t cb = s_base[l] + m;
-                const uint32_t s0 = a.cell_start[cb], e = a.cell_start[cb + 1];
-                if (e > s0) {
-                  if (l > L0 && e - s0 > a.tree_leaf) {
-                    down = true;
-                  } else {
-                    // A leaf of more than one chunk goes chunk by chunk: a
-                    // chunk whose box lies beyond the limit (with the cells'
-                    // FP32 margin) holds no hit.
-                    const bool chunked = a.chunk_box && e - s0 > kChunkPts;
-                    for (uint32_t c0 = s0; c0 < e;) {
-                      uint32_t c1 = e;
-                      if (chunked) {
-                        const uint32_t ch = c0 / kChunkPts;
-                        c1 = min(e, (ch + 1) * kChunkPts);
-                        const float4 blo = a.chunk_box[2 * ch], bhi = a.chunk_box[2 * ch + 1];
-                        const float bx = fmaxf(fmaxf(blo.x - qv.x, qv.x - bhi.x), 0.0f);
-                        const float by = fmaxf(fmaxf(blo.y - qv.y, qv.y - bhi.y), 0.0f);
-                        const float bz = fmaxf(fmaxf(blo.z - qv.z, qv.z - bhi.z), 0.0f);
-                        if ((bx * bx + by * by) + bz * bz > lim * 1.001f) {
-                          c0 = c1;
-                          continue;
-                        }
-                      }
-                      for (uint32_t j = c0; j < c1; ++j) {
-                        const float4 p = a.spts[j];
-                        const float d2 = d2_of(qv.x, qv.y, qv.z, p.x, p.y, p.z);
-                        if (d2 > 0.0f && d2 <= lim) {
-                          const uint64_t key = pack_key(d2, __float_as_uint(p.w));
-                          if (key < list[KC - 1]) {
-                            topk_insert<KC>(list, key);
-                            if (list[KC - 1] != ~0ull) lim = fminf(lim, key_d2(list[KC - 1]));
-                          }
-                        }
-                      }
-                      c0 = c1;
-                    }
-                  }
-                }
-              }
-              if (down) {
-                --l;
-                m = (m << 3) | ((qm >> (3 * l)) & 7u);
-                continue;
-              }
-              // next sibling in visiting order, climbing past last children
-              while (l < T && (((m & 7u) ^ ((qm >> (3 * l)) & 7u)) == 7u)) {
-                m >>= 3;
-                ++l;
-              }
-              if (l == T) break;
-              const uint32_t o = (qm >> (3 * l)) & 7u;
-              m = (m & ~7u) | ((((m & 7u) ^ o) + 1u) ^ o);
-            }
-          }
-    }
-    const uint32_t k = a.k;
-    const uint32_t base = a.local_index ? g0.point_base : 0u;
-    int32_t* oi = a.out_idx + (uint64_t)row * k;
-    float* od = a.out_d2 ? a.out_d2 + (uint64_t)row * k : nullptr;
-    uint32_t hits = 0;
-#pragma unroll
-    for (int i = 0; i < KC; ++i) {
-      if ((uint32_t)i < k) {
-        const bool have = list[i] != ~0ull;
-        hits += have ? 1u : 0u;
-        oi[i] = have ? (int32_t)(key_idx(list[i]) - base) : -1;
-        if (od) od[i] = have ? key_d2(list[i]) : __builtin_huge_valf();
-      }
-    }
-    if (a.short_rows) append_short(a, hits < k && R < a.r, qs, hits, R);
-  }
-}
-
-// --------------------------------------------------------------------------
-// The octree walk with G lanes per query
-//
-// k_topk_tree walks one query per lane; a walk that crosses a dense cluster
-// scans its leaves chunk after chunk on that one lane while the L2 latency of
-// every load is exposed (the Levy-flight KNN: 0.30 of the VALU slots, 97 %
-// L2 hits).  Here the G lanes of a group walk the same octree path -- every
-// decision reads a limit the group shares, so their control flow is the
-// same -- and deal each leaf's chunks to them round-robin (lane l tests and
-// scans chunks l, l + G, ...; a leaf of one chunk has its points split), each
-// into a top-k list of its own.  After each round the group takes the
-// smallest of its lanes' limits: once a lane holds
-// k keys with d2 <= t, no point beyond t is among the group's k nearest, so
-// every lane may prune at the smallest lane limit.  At the end the G sorted
-// lists are merged by repeatedly taking the group's smallest head (the
-// points of one list are distinct from every other's, so each head is
-// unique); the row is the first k taken.  Same result as k_topk_tree.
-// On the Levy-flight KNN (30M x 30M, leaves of 65536 points; builds without
-// occupancy targets: two waves per SIMD for one lane, three for several) one
-// lane took 1080 ms, two lanes 900 ms, four 1062 ms, eight 1245 ms: beyond
-// two, the walk every lane repeats (cell bounds, boxes) outweighs the split
-// chunks.
-
-template <int G>
-__device__ inline float group_min_f(float v) {
-#pragma unroll
-  for (int o = 1; o < G; o <<= 1) v = fminf(v, __shfl_xor(v, o, G));
-  return v;
-}
-
-template <int G>
-__device__ inline uint64_t group_min_u64(uint64_t v) {
-#pragma unroll
-  for (int o = 1; o < G; o <<= 1) {
-    const uint64_t w = (uint64_t)__shfl_xor((unsigned long long)v, o, G);
-    v = w < v ? w : v;
-  }
-  return v;
-}
-
-template <int KC, int G>
-__global__ __launch_bounds__(kTileQ) __attribute__((amdgpu_waves_per_eu(treeg_waves<KC>())))
-void k_topk_treeg(const SearchArgs a) {
-  __shared__ uint32_t s_base[8];
-  if (threadIdx.x < 8) s_base[threadIdx.x] = (int)threadIdx.x < a.nlevels ?
-                                               a.grids[threadIdx.x].cell_base : 0u;
-  __syncthreads();
-  const uint32_t nq = launch_nq(a);
-  const int T = a.nlevels - 1, L0 = a.level_min;
-  const GridDesc g0 = a.grids[0];
-  const int gq = threadIdx.x / G, l = threadIdx.x % G;
-  for (TileIter it(a, nq); it.t < it.end; it.t += it.step) {
-    uint32_t q0, q1, gi;
-    tile_of(a, nq, it.t, q0, q1, gi);
-    const uint32_t qi = q0 + gq;
-    if (qi >= q1) continue;  // the whole group
-    const uint32_t qs = a.qsel ? a.qsel[qi] : qi;
-    const float4 qv = a.queries[qs];
-    const uint32_t row = __float_as_uint(qv.w);
-    const float R = query_radius(a, qi, qs);
-    float lim = r2_limit(R * R);
-    uint64_t list[KC];
-#pragma unroll
-    for (int i = 0; i < KC; ++i) list[i] = ~0ull;
-    // points j0, j0 + step, ... < j1 into the lane's list
-    auto scan = [&](uint32_t j0, uint32_t j1, uint32_t step) {
-      for (uint32_t j = j0; j < j1; j += step) {
-        const float4 p = a.spts[j];
-        const float d2 = d2_of(qv.x, qv.y, qv.z, p.x, p.y, p.z);
-        if (d2 > 0.0f && d2 <= lim) {
-          const uint64_t key = pack_key(d2, __float_as_uint(p.w));
-          if (key < list[KC - 1]) {
-            topk_insert<KC>(list, key);
-            if (list[KC - 1] != ~0ull) lim = fminf(lim, key_d2(list[KC - 1]));
-          }
-        }
-      }
-    };
-    int lo0, hi0, lo1, hi1, lo2, hi2;
-    cell_range(g0, qv.x, R, 0, lo0, hi0);
-    cell_range(g0, qv.y, R, 1, lo1, hi1);
-    cell_range(g0, qv.z, R, 2, lo2, hi2);
-    const int qc0 = min(max((int)floorf((qv.x - g0.mn[0]) * g0.inv), 0), g0.dim[0] - 1);
-    const int qc1 = min(max((int)floorf((qv.y - g0.mn[1]) * g0.inv), 0), g0.dim[1] - 1);
-    const int qc2 = min(max((int)floorf((qv.z - g0.mn[2]) * g0.inv), 0), g0.dim[2] - 1);
-    const uint32_t qm = morton3((uint32_t)qc0, (uint32_t)qc1, (uint32_t)qc2);
-    const float mag = fabsf(g0.mn[0]) + fabsf(g0.mn[1]) + fabsf(g0.mn[2]) + fabsf(qv.x) +
-                      fabsf(qv.y) + fabsf(qv.z) + (float)g0.dim[0] * g0.cell;
-    if (hi0 >= lo0 && hi1 >= lo1 && hi2 >= lo2) {
-      const int tl0 = lo0 >> T, th0 = hi0 >> T, tl1 = lo1 >> T, th1 = hi1 >> T;
-      const int tl2 = lo2 >> T, th2 = hi2 >> T;
-      const int qt0 = qc0 >> T, qt1 = qc1 >> T, qt2 = qc2 >> T;
-      const int nring = max(max(max(qt0 - tl0, th0 - qt0), max(qt1 - tl1, th1 - qt1)),
-                            max(qt2 - tl2, th2 - qt2));
-      for (int ring = 0; ring <= nring; ++ring)
-      for (int tz = max(tl2, qt2 - ring); tz <= min(th2, qt2 + ring); ++tz)
-        for (int ty = max(tl1, qt1 - ring); ty <= min(th1, qt1 + ring); ++ty)
-          for (int tx = max(tl0, qt0 - ring); tx <= min(th0, qt0 + ring); ++tx) {
-            if (max(max(abs(tx - qt0), abs(ty - qt1)), abs(tz - qt2)) != ring) continue;
-            int lv = T;
-            uint32_t m = morton3((uint32_t)tx, (uint32_t)ty, (uint32_t)tz);
-            for (;;) {
-              const float c = ldexpf(g0.cell, lv);
-              const float pad = c * 0x1.0p-12f + mag * 0x1.0p-19f;
-              const float bd = box_d2(qv, g0, c, pad, compact3(m), compact3(m >> 1),
-                                      compact3(m >> 2));
-              bool down = false;
-              if (bd <= lim * 1.001f) {
-                const uint32_t cb = s_base[lv] + m;
-                const uint32_t s0 = a.cell_start[cb], e = a.cell_start[cb + 1];
-                if (e > s0) {
-                  if (lv > L0 && e - s0 > a.tree_leaf) {
-                    down = true;
-                  } else if (a.chunk_box && e - s0 > kChunkPts) {
-                    // the leaf's chunks dealt round-robin to the lanes, each
-                    // tested against its box and scanned by its lane; the
-                    // group's limit after every round
-                    const uint32_t first = s0 / kChunkPts, last = (e - 1) / kChunkPts;
-                    for (uint32_t cr = first; cr <= last; cr += G) {
-                      const uint32_t ch = cr + (uint32_t)l;
-                      if (ch <= last) {
-                        const float4 blo = a.chunk_box[2 * ch], bhi = a.chunk_box[2 * ch + 1];
-                        const float bx = fmaxf(fmaxf(blo.x - qv.x, qv.x - bhi.x), 0.0f);
-                        const float by = fmaxf(fmaxf(blo.y - qv.y, qv.y - bhi.y), 0.0f);
-                        const float bz = fmaxf(fmaxf(blo.z - qv.z, qv.z - bhi.z), 0.0f);
-                        if ((bx * bx + by * by) + bz * bz <= lim * 1.001f)
-                          scan(max(s0, ch * kChunkPts), min(e, (ch + 1) * kChunkPts), 1u);
-                      }
-                      lim = group_min_f<G>(lim);
-                    }
-                  } else {
-                    scan(s0 + (uint32_t)l, e, G);  // a small leaf: its points split
-                    lim = group_min_f<G>(lim);
-                  }
-                }
-              }
-              if (down) {
-                --lv;
-                m = (m << 3) | ((qm >> (3 * lv)) & 7u);
-                continue;
-              }
-              while (lv < T && (((m & 7u) ^ ((qm >> (3 * lv)) & 7u)) == 7u)) {
-                m >>= 3;
-                ++lv;
-              }
-              if (lv == T) break;
-              const uint32_t o = (qm >> (3 * lv)) & 7u;
-              m = (m & ~7u) | ((((m & 7u) ^ o) + 1u) ^ o);
-            }
-          }
-    }
-    // merge: the group's smallest head, k times
-    const uint32_t k = a.k;
-    const uint32_t base = a.local_index ? g0.point_base : 0u;
-    int32_t* oi = a.out_idx + (uint64_t)row * k;
-    float* od = a.out_d2 ? a.out_d2 + (uint64_t)row * k : nullptr;
-    uint32_t hits = 0;
-#pragma unroll
-    for (int i = 0; i < KC; ++i) {
-      if ((uint32_t)i < k) {
-        const uint64_t m = group_min_u64<G>(list[0]);
-        const bool have = m != ~0ull;
-        hits += have ? 1u : 0u;
-        if (l == i % G) {
-          oi[i] = have ? (int32_t)(key_idx(m) - base) : -1;
-          if (od) od[i] = have ? key_d2(m) : __builtin_huge_valf();
-        }
-        const bool win = have && list[0] == m;
-#pragma unroll
-        for (int j = 0; j < KC - 1; ++j) list[j] = win ? list[j + 1] : list[j];
-        list[KC - 1] = win ? ~0ull : list[KC - 1];
-      }
-    }
-    if (a.short_rows) append_short(a, l == 0 && hits < k && R < a.r, qs, hits, R);
   }
 }
 
@@ -916,7 +518,10 @@ __global__ __launch_bounds__(kTileQ) void k_topk_group(const SearchArgs a) {
       cell_range(g, qv.y, R, 1, lo1, hi1);
       cell_range(g, qv.z, R, 2, lo2, hi2);
       uint32_t lvl_base = g.cell_base;
-      if (HIER) {  // same level rule as k_topk_thread (group-uniform)
+      if (HIER) {
+        // Finest built level whose cell is >= R * alpha (group-uniform); the
+        // level-0 range shifted right by the level is that level's range (floor
+        // division is monotone and keeps empty ranges empty).
         int lvl = a.level_min;
         float c = ldexpf(g.cell, lvl);
         const float want = R * a.level_alpha;
@@ -1525,21 +1130,10 @@ __global__ __launch_bounds__(kTileQ) void k_topk_tiled(const SearchArgs a) {
 
 template <int KC>
 static void launch_thread(const SearchArgs& a, bool knn, dim3 grid, hipStream_t st) {
-  const bool hier = a.nlevels > 0;
-  if (knn && hier && a.tree_lanes == 2)
-    hipLaunchKernelGGL((k_topk_treeg<KC, 2>), grid, dim3(kTileQ), 0, st, a);
-  else if (knn && hier && a.tree_lanes == 4)
-    hipLaunchKernelGGL((k_topk_treeg<KC, 4>), grid, dim3(kTileQ), 0, st, a);
-  else if (knn && hier && a.tree_lanes == 8)
-    hipLaunchKernelGGL((k_topk_treeg<KC, 8>), grid, dim3(kTileQ), 0, st, a);
-  else if (knn && hier)
-    hipLaunchKernelGGL((k_topk_tree<KC>), grid, dim3(kTileQ), 0, st, a);
-  else if (knn)
-    hipLaunchKernelGGL((k_topk_thread<KC, true, false>), grid, dim3(kTileQ), 0, st, a);
-  else if (hier)
-    hipLaunchKernelGGL((k_topk_thread<KC, false, true>), grid, dim3(kTileQ), 0, st, a);
+  if (knn)
+    hipLaunchKernelGGL((k_topk_thread<KC, true>), grid, dim3(kTileQ), 0, st, a);
   else
-    hipLaunchKernelGGL((k_topk_thread<KC, false, false>), grid, dim3(kTileQ), 0, st, a);
+    hipLaunchKernelGGL((k_topk_thread<KC, false>), grid, dim3(kTileQ), 0, st, a);
 }
 
 template <int G, int KB, int TP>
@@ -1568,8 +1162,6 @@ static void launch_group(const SearchArgs& a, bool knn, bool wide, int tile, dim
     hipLaunchKernelGGL((k_topk_group<G, KB, true, false, true>), grid, dim3(kTileQ), 0, st, a);
   else if (knn)
     hipLaunchKernelGGL((k_topk_group<G, KB, true, false, false>), grid, dim3(kTileQ), 0, st, a);
-  else if (hier)
-    hipLaunchKernelGGL((k_topk_group<G, KB, false, true, true>), grid, dim3(kTileQ), 0, st, a);
   else if (wide)
     hipLaunchKernelGGL((k_topk_group<G, KB, false, false, true>), grid, dim3(kTileQ), 0, st, a);
   else
@@ -1642,16 +1234,13 @@ hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hi
     return launch_search(o, knn_mode, 4, st, num_cus, true, 0, true, 0);
   }
   if (k == 0 || k > max_k_for_group(group_lanes)) return hipErrorInvalidValue;
+  // hierarchical grids: KNN by groups (one lane per query is the packet walk's)
+  if (a.nlevels > 0 && (group_lanes == 1 || !knn_mode)) return hipErrorInvalidValue;
   if (!a.tiles) {
     // Implicit tiles: a block of the thread kernel takes kTileQ queries, a
     // block of the group kernel one query per group, so small workloads still
     // spread over many blocks.
-    // the octree walk with several lanes per query takes kTileQ / lanes
-    // queries per block, as a group kernel does
-    const bool tree_g = group_lanes == 1 && knn_mode != 0 && a.nlevels > 0 &&
-                        (a.tree_lanes == 2 || a.tree_lanes == 4 || a.tree_lanes == 8);
-    a.tile_q = tree_g ? (uint32_t)(kTileQ / a.tree_lanes)
-                      : group_lanes == 1 ? (uint32_t)kTileQ : (uint32_t)(kTileQ / group_lanes);
+    a.tile_q = (uint32_t)(kTileQ / group_lanes);
     a.ntiles = (uint32_t)(((uint64_t)a.nq + a.tile_q - 1) / a.tile_q);
   }
   if (a.ntiles == 0) return hipSuccess;
