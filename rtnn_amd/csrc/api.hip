@@ -206,6 +206,8 @@ struct rtnn_ctx_s {
   DevBuf pts;
   uint64_t n = 0;
   float bbox[6] = {0, 0, 0, 0, 0, 0};
+  DevBuf bbox_tmp;
+  PinBuf pbbox;
 
   // grid
   DevBuf keys, vals, counts, cell_start, spts, tmp, grids;
@@ -266,8 +268,9 @@ struct rtnn_ctx_s {
                      &qin, &qkeys, &qvals, &qsorted, &oidx, &od2, &shortrows, &misc,
                      &tiles, &offs, &bboxes, &pgrid, &pcounts, &qradius, &tr_q, &tr_idx,
                      &tr_d2, &tr_t, &tr_f, &tr_out, &bcnt, &boff, &bpairs, &ovf,
-                     &boxes};
+                     &boxes, &bbox_tmp};
     for (DevBuf* b : all) b->release();
+    pbbox.release();
     if (st3) (void)hipStreamSynchronize(st3);
     for (int i = 0; i < 2; ++i) {
       sq[i].release();
@@ -409,6 +412,22 @@ int clear_counts(rtnn_ctx ctx, uint64_t ncells) {
 }
 void grid_built(rtnn_ctx ctx, uint64_t ncells, uint64_t was_zero) {
   ctx->counts_zero = std::max(ncells, was_zero);
+}
+
+// Whether a kernel on `device` may read `bytes` at p itself: whole floats inside
+// one of this device's allocations.
+bool readable_here(int device, const void* p, uint64_t bytes) {
+  hipPointerAttribute_t attr;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess ||
+      hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const uintptr_t at = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(base);
+  return attr.type == hipMemoryTypeDevice && attr.device == device && at % 4 == 0 && at >= b &&
+         bytes <= size && at - b <= size - bytes;
 }
 
 // Builds the single-cloud grid over ctx->pts with edge `cell` (grown until the
@@ -896,25 +915,28 @@ int rtnn_set_points(rtnn_ctx ctx, const float* xyz, uint64_t n, int on_device) {
   if (!xyz) return fail(ctx, RTNN_ERR_INVALID, "xyz is NULL");
   if (n >= 0xffffffffull) return fail(ctx, RTNN_ERR_UNSUPPORTED, "more than 2^32-2 points");
   CK(hipSetDevice(ctx->device));
+  if (!ctx->bbox_tmp.p) {  // the reduction's ticket word, then its partial boxes
+    CK(ctx->bbox_tmp.ensure(256 + kBboxPartBytes));
+    CK(fill_u32(ctx->bbox_tmp.as<uint32_t>(), 1, 0, ctx->st));
+  }
+  CK(ctx->pbbox.ensure(64));
   CK(ctx->pts.ensure(12 * n));
-  CK(hipMemcpyAsync(ctx->pts.p, xyz, 12 * n,
-                    on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->st));
+  // Points on this device are copied by the kernel that reduces them; others
+  // (host memory, another device's) by the runtime before it.
+  const bool fused = on_device && readable_here(ctx->device, xyz, 12 * n);
+  if (!fused)
+    CK(hipMemcpyAsync(ctx->pts.p, xyz, 12 * n,
+                      on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->st));
   ctx->n = n;
   ctx->spts_current = false;
-  CK(ctx->misc.ensure(4096 + 6 * 4 * kBboxBlocks));
-  float* bb = ctx->misc.as<float>();
-  uint32_t* bad = reinterpret_cast<uint32_t*>(bb + 8);
-  float* part = bb + 16;
-  CK(fill_u32(bad, 1, 0, ctx->st));
-  CK(bbox(ctx->pts.as<float>(), n, part, bb, bad, ctx->st));
-  float hb[16];
-  CK(hipMemcpyAsync(hb, bb, 64, hipMemcpyDeviceToHost, ctx->st));
+  float* hb = static_cast<float*>(ctx->pbbox.p);
+  uint32_t* bad = reinterpret_cast<uint32_t*>(hb + 8);
+  CK(bbox(fused ? xyz : ctx->pts.as<float>(), fused ? ctx->pts.as<float>() : nullptr, n,
+          ctx->bbox_tmp.as<float>() + 64, ctx->bbox_tmp.as<uint32_t>(), hb, bad, ctx->st));
   CK(hipStreamSynchronize(ctx->st));
-  uint32_t nbad;
-  std::memcpy(&nbad, &hb[8], 4);
-  if (nbad) {
+  if (*bad) {
     ctx->n = 0;
-    return fail(ctx, RTNN_ERR_INVALID, "%u non-finite point coordinates", nbad);
+    return fail(ctx, RTNN_ERR_INVALID, "%u non-finite point coordinates", *bad);
   }
   std::memcpy(ctx->bbox, hb, sizeof ctx->bbox);
   return RTNN_OK;
@@ -952,7 +974,10 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
   rc = prepare_queries(ctx, qxyz, nq, on_device, &qproc,
                        packet ? kPacketKeyBits : kQueryKeyBits);
   if (rc) return rc;
-  if (timing) CK(hipEventRecord(ctx->ev[2], ctx->st));
+  // A stage that does nothing takes no event: each costs a small call several us.
+  const hipEvent_t ev_sorted = qxyz ? ctx->ev[2] : ctx->ev[1];
+  const hipEvent_t ev_copied = out_on_device ? ctx->ev[3] : ctx->ev[4];
+  if (timing && qxyz) CK(hipEventRecord(ev_sorted, ctx->st));
   OutBufs o;
   rc = output_targets(ctx, nq, k, out_idx, out_d2, out_on_device, o);
   if (rc) return rc;
@@ -970,15 +995,15 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
   rc = copy_out(ctx, nq, k, out_idx, out_d2, out_on_device, o);
   if (rc) return rc;
   if (!wait) return RTNN_OK;
-  if (timing) CK(hipEventRecord(ctx->ev[4], ctx->st));
+  if (timing && !out_on_device) CK(hipEventRecord(ev_copied, ctx->st));
   CK(hipStreamSynchronize(ctx->st));
   if (stats) {
     std::memset(stats, 0, sizeof *stats);
     stats->ms_grid = ev_ms(ctx->ev[0], ctx->ev[1]);
-    stats->ms_qsort = ev_ms(ctx->ev[1], ctx->ev[2]);
-    stats->ms_search = ev_ms(ctx->ev[2], ctx->ev[3]);
-    stats->ms_copy = out_on_device ? 0.0 : ev_ms(ctx->ev[3], ctx->ev[4]);
-    stats->ms_total = ev_ms(ctx->ev[0], ctx->ev[4]);
+    stats->ms_qsort = qxyz ? ev_ms(ctx->ev[1], ev_sorted) : 0.0;
+    stats->ms_search = ev_ms(ev_sorted, ctx->ev[3]);
+    stats->ms_copy = out_on_device ? 0.0 : ev_ms(ctx->ev[3], ev_copied);
+    stats->ms_total = ev_ms(ctx->ev[0], ev_copied);
     stats->search_launches = pooled ? 2 : 1;
     stats->lanes_per_query = pooled ? (uint32_t)(64 / ctx->opt.queries_per_wave) : (uint32_t)gl;
     fill_stats(ctx, stats);
@@ -1048,7 +1073,7 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
     used += (bytes + 255) & ~255ull;
     return at;
   };
-  const uint64_t o_status = take(16), o_offs = take(16), o_part = take(4 * 6 * kBboxBlocks);
+  const uint64_t o_status = take(16), o_offs = take(16), o_part = take(kBboxPartBytes);
   const uint64_t o_bb = take(4 * 6), o_grid = take(sizeof(GridDesc));
   const uint64_t o_keys = take(4 * n), o_vals = take(4 * n);
   const uint64_t o_spts = take(16 * n + kSptsPadBytes);
@@ -1082,12 +1107,14 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
   uint32_t* cell_start = reinterpret_cast<uint32_t*>(base + o_cells);
   CK(hipSetDevice(ctx->device));
   hipStream_t st = ctx->st;
-  // status: [0] non-finite coordinates, [1] planning fell back, [2] cells;
+  // status: [0] non-finite coordinates, [1] planning fell back, [2] cells,
+  // [3] the box reduction's ticket;
   // offsets of the one cloud: {0, n}
   CK(fill_u32(status, 4, 0, st));
   CK(fill_u32(reinterpret_cast<uint32_t*>(offs), 4, 0, st));
   CK(fill_u32(reinterpret_cast<uint32_t*>(offs) + 2, 1, (uint32_t)n, st));
-  CK(bbox(xyz, n, reinterpret_cast<float*>(base + o_part), bb, &status[0], st));
+  CK(bbox(xyz, nullptr, n, reinterpret_cast<float*>(base + o_part), &status[3], bb, &status[0],
+          st));
   const float f = ctx->opt.cell_factor > 0 ? ctx->opt.cell_factor : default_cell_factor(mode);
   CK(plan_batched(bb, offs, 1, r / f, nullptr, cap, grid, status, st));
   CK(cell_keys(xyz, n, grid, offs, 1, keys, vals, nullptr, st));
@@ -1940,13 +1967,14 @@ int build_batched(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets, uint3
   // Per-cloud bbox on the device, plan on the host.
   CK(ctx->offs.ensure(8 * (nclouds + 1)));
   CK(hipMemcpyAsync(ctx->offs.p, offsets, 8 * (nclouds + 1), hipMemcpyHostToDevice, ctx->st));
-  CK(ctx->bboxes.ensure(24 * nclouds + 64 + (nclouds == 1 ? 4 * 6 * kBboxBlocks : 0)));
+  CK(ctx->bboxes.ensure(24 * nclouds + 64 + (nclouds == 1 ? kBboxPartBytes : 0)));
   uint32_t* bad = reinterpret_cast<uint32_t*>(ctx->bboxes.as<float>() + 6 * nclouds);
-  CK(fill_u32(bad, 1, 0, ctx->st));
+  CK(fill_u32(bad, 2, 0, ctx->st));  // the count and the reduction's ticket
   if (nclouds == 1)  // one cloud: the multi-block reduction (partials after the box)
-    CK(bbox(xyz, n, ctx->bboxes.as<float>() + 16, ctx->bboxes.as<float>(), bad, ctx->st));
+    CK(bbox(xyz, nullptr, n, ctx->bboxes.as<float>() + 16, bad + 1, ctx->bboxes.as<float>(), bad,
+            ctx->st));
   else
-    CK(bbox_segmented(xyz, ctx->offs.as<uint64_t>(), nclouds, ctx->bboxes.as<float>(), bad,
+    CK(bbox_segmented(xyz, ctx->offs.as<uint64_t>(), nclouds, n, ctx->bboxes.as<float>(), bad,
                       ctx->st));
   std::vector<float> hb(6 * nclouds + 1);
   CK(hipMemcpyAsync(hb.data(), ctx->bboxes.p, 4 * (6 * nclouds + 1), hipMemcpyDeviceToHost,
@@ -2748,9 +2776,10 @@ hipError_t enqueue_batched(rtnn_graph g, const float* xyz, float cell, int mode,
   // One cloud: the multi-block reduction (the per-cloud kernel gives each
   // cloud one block, which for a single large cloud is the slowest step).
   if (g->nclouds == 1)
-    e = bbox(xyz, g->n, g->bbox_part.as<float>(), g->bboxes.as<float>(), status, st);
+    e = bbox(xyz, nullptr, g->n, g->bbox_part.as<float>(), &status[3], g->bboxes.as<float>(),
+             status, st);
   else
-    e = bbox_segmented(xyz, off, g->nclouds, g->bboxes.as<float>(), status, st);
+    e = bbox_segmented(xyz, off, g->nclouds, g->n, g->bboxes.as<float>(), status, st);
   if (e != hipSuccess) return e;
   const float* cells = g->class_opt.empty() ? nullptr : g->ccells.as<float>();
   if ((e = plan_batched(g->bboxes.as<float>(), off, g->nclouds, cell, cells, g->cap_cells,
@@ -2850,7 +2879,7 @@ int rtnn_graph_batched(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets,
   }
   CK(g->tiles.ensure(sizeof(Tile) * g->ntiles));
   CK(g->ccells.ensure(4 * (uint64_t)nclouds));
-  if (nclouds == 1) CK(g->bbox_part.ensure(4 * 6 * kBboxBlocks));
+  if (nclouds == 1) CK(g->bbox_part.ensure(kBboxPartBytes));
   CK(hipMemcpyAsync(g->ccells.p, cells.data(), 4 * (uint64_t)nclouds, hipMemcpyHostToDevice,
                     ctx->st));
   CK(hipMemcpyAsync(g->offs.p, offsets, 8 * (nclouds + 1), hipMemcpyHostToDevice, ctx->st));

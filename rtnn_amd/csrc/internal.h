@@ -20,12 +20,15 @@ hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint64_t n, int bits
 
 // ---- grid.hip
 constexpr int kBboxBlocks = 1024;
-// part: 6 * kBboxBlocks floats; out: 6 floats (min xyz, max xyz); nonfinite: 1 u32.
-hipError_t bbox(const float* xyz, uint64_t n, float* part, float* out, uint32_t* nonfinite,
-                hipStream_t st);
-// Per-cloud bbox: out[6 * c .. 6 * c + 6) for cloud c (offsets: nclouds + 1).
+constexpr uint64_t kBboxPartBytes = 4 * 8 * kBboxBlocks;
+// Copies the points to dst (unless null) and reduces them.  part: kBboxPartBytes;
+// *ticket: 0 before and after; out: 6 floats (min xyz, max xyz); nonfinite: 1 u32.
+// out and nonfinite may be pinned host memory.
+hipError_t bbox(const float* src, float* dst, uint64_t n, float* part, uint32_t* ticket,
+                float* out, uint32_t* nonfinite, hipStream_t st);
+// Per-cloud bbox: out[6 * c .. 6 * c + 6) for cloud c (offsets: nclouds + 1, n points in all).
 hipError_t bbox_segmented(const float* xyz, const uint64_t* offsets, uint32_t nclouds,
-                          float* out, uint32_t* nonfinite, hipStream_t st);
+                          uint64_t n, float* out, uint32_t* nonfinite, hipStream_t st);
 // Per-cloud grids planned on the device from the per-cloud bboxes: edge
 // cells[i] (device array, size classes) or `cell` when cells is null, every
 // edge grown by the same 1.25x steps until the total cell count is <= cap
