@@ -178,6 +178,7 @@ def timed(fn, steps, warmup, label):
            for f in ("ms_total", "ms_grid", "ms_qsort", "ms_search", "ms_mlp", "ms_fallback")}
     agg["fallback_queries"] = int(stats[-1].fallback_queries)
     agg["lanes_per_query"] = int(stats[-1].lanes_per_query)
+    agg["grid_dims"] = list(stats[-1].grid_dims)
     agg["cell_size"] = float(stats[-1].cell_size)
     agg["sort_passes"] = int(stats[-1].sort_passes)
     log(f"[bench] {label}: {steps} steps, {ms:.3f} ms/step; " +
@@ -247,6 +248,8 @@ def kernel_name(res, mode, opts, method):
     """Name of the dominant search kernel of a method's configuration."""
     o = opts or {}
     if res.get("lanes_per_query") == 1 and not o.get("group_buffer") == 3:
+        if mode == "knn" and method == "plain" and list(res.get("grid_dims", ())) != [1024] * 3:
+            return "k_topk_thread"
         if mode == "knn" and (method == "plain" or o.get("grid_levels", 0) >= 2 or
                               (method == "partitioned" and not o.get("grid_levels"))):
             return "k_knn_packet"

@@ -430,11 +430,20 @@ bool readable_here(int device, const void* p, uint64_t bytes) {
          bytes <= size && at - b <= size - bytes;
 }
 
-// Builds the single-cloud grid over ctx->pts with edge `cell` (grown until the
-// cell count fits the budget).  desc_event: separate queries follow, ordered on
-// the second stream as soon as the descriptor is on the device.
-int build_grid(rtnn_ctx ctx, float cell, bool desc_event = true) {
-  GridDesc g;
+// The bounding-box reduction's buffers, which the cell spread shares.
+int ensure_reduction(rtnn_ctx ctx) {
+  static_assert(kSpreadDraws / 256 * 16 <= kBboxPartBytes, "16 bytes per block");
+  if (!ctx->bbox_tmp.p) {  // the ticket word, then the partial results
+    CK(ctx->bbox_tmp.ensure(256 + kBboxPartBytes));
+    CK(fill_u32(ctx->bbox_tmp.as<uint32_t>(), 1, 0, ctx->st));
+  }
+  CK(ctx->pbbox.ensure(64));
+  return RTNN_OK;
+}
+
+// The single-cloud grid over ctx->pts with edge `cell`, grown until the cell
+// count fits the budget.
+int plan_single(rtnn_ctx ctx, float cell, GridDesc& g) {
   const uint64_t cap = max_cells_for(ctx, ctx->n);
   for (int tries = 0;; ++tries) {
     plan_grid(ctx->bbox, cell, g);
@@ -445,6 +454,91 @@ int build_grid(rtnn_ctx ctx, float cell, bool desc_event = true) {
   g.cell_base = 0;
   g.point_base = 0;
   g.npoints = (uint32_t)ctx->n;
+  return RTNN_OK;
+}
+
+// Lanes per query for a KNN over the cells of edge r (1, 4 or 16), 0 for the
+// packet walk.  mean: points in a point's cell, itself included, on average;
+// skew: how much more the fuller cells hold (1 to 1.25 on uniform points, 3 and
+// more on clusters, where the fullest cells would hold up the chip alone).
+//
+// A packet of 64 neighbouring queries reaches several times the points that any
+// one of them has in its 27 cells, so where few points share a cell the cells
+// win; few queries do not fill the chip with packets, and 16 lanes each do.  The
+// lines lie where the two meet (us per pass over all points, packets / one lane
+// / 4 lanes / 16 lanes):
+//   10k points   mean 2.3, K = 8    123 /  64 /  39 /  37;  mean 34   180 / 282 / 235 / 82
+//                mean 51, K = 64    281 /   - /   - / 209;  mean 150  302 /   - /   - / 375
+//   100k         mean 2.4, K = 16   169 /  93 /  64 /  78;  mean 7.4  193 / 160 / 171 / 95
+//                mean 16, K = 32    212 / 485 / 642 / 172;  mean 36   234 / 757 / 1362 / 419
+//   1M, K = 4    mean 2.4           344 / 183 / 231 / 394;  mean 12   432 / 325 / 1121 / 925
+//       K = 16   mean 2.4           486 / 327 / 237 / 393;  mean 7.4  607 / 618 / 1047 / 620
+//       K = 64   mean 2.4          1661 / 2512 / 351 / 436; mean 12  2415 / 8625 / 689 / 826
+//                mean 33           2349 / 10768 / 14788 / 3921
+//       K = 8    clusters, mean 7   489 / 1175 / 1609 / 1366
+int knn_cell_lanes(uint64_t nq, uint32_t k, double mean, double skew) {
+  if (nq <= 1ull << 14) return mean <= 64.0 ? 16 : 0;
+  if (skew > 3.0) return 0;
+  if (nq <= 1ull << 17) return mean <= 3.0 ? 4 : mean <= 24.0 ? 16 : 0;
+  if (k <= 8) return mean <= 16.0 ? 1 : 0;
+  if (k <= 16) return mean <= 4.0 ? 4 : mean <= 8.0 && nq <= 1ull << 19 ? 16 : 0;
+  if (k <= 32) return mean <= 8.0 ? 4 : mean <= 12.0 ? 16 : 0;
+  return mean <= 12.0 ? 4 : mean <= 20.0 ? 16 : 0;
+}
+constexpr double kMostMean = 64.0;  // beyond it knn_cell_lanes is 0
+
+// Measures the cells of edge r and sets *lanes to knn_cell_lanes; waits for the
+// device (one launch and the wait: about 20 us, which a search that may not wait
+// does without, by packets).  Spares itself that where even evenly spread points
+// would be too many per cell.
+int probe_cells(rtnn_ctx ctx, float r, uint64_t nq, uint32_t k, int* lanes) {
+  *lanes = 0;
+  GridDesc g;
+  if (plan_single(ctx, r, g)) return RTNN_OK;  // no such grid: by packets
+  const uint64_t n = ctx->n, ncells = grid_cells(g);
+  if ((double)n > kMostMean * (double)ncells) return RTNN_OK;
+  const int re = ensure_reduction(ctx);
+  if (re) return re;
+  const uint32_t m = (uint32_t)std::min<uint64_t>(n, kSpreadDraws);
+  const int tbits = std::max(12, bits_for(8ull * m - 1));
+  const uint64_t words = 1ull << tbits;
+  const bool hashed = ncells > words;
+  const uint64_t zero = ctx->counts_zero;
+  const int rz = clear_counts(ctx, words);
+  if (rz) return rz;
+  CellSpread* s = static_cast<CellSpread*>(ctx->pbbox.p);
+  CK(cell_spread(ctx->pts.as<float>(), n, m, g, hashed, tbits, ctx->counts.as<uint32_t>(),
+                 reinterpret_cast<uint64_t*>(ctx->bbox_tmp.as<uint32_t>() + 64),
+                 ctx->bbox_tmp.as<uint32_t>(), s, ctx->st));
+  CK(hipStreamSynchronize(ctx->st));
+  CK(fill_u32(ctx->counts.as<uint32_t>(), words, 0, ctx->st));
+  grid_built(ctx, words, zero);
+  // Draws that only share a slot of the table are taken off by their expected
+  // number; then sums of c^2 and c^3 over the cells, per point.
+  const double t = (double)words, md = (double)m, nd = (double)n;
+  double pairs = (double)s->pairs, triples = (double)s->triples;
+  if (hashed) {
+    pairs = std::max(0.0, pairs - md * md / (2.0 * t));
+    triples = std::max(0.0, triples - pairs * md / t - md * md * md / (6.0 * t * t));
+  }
+  double mean, cube;
+  if (m == n) {
+    mean = 1.0 + 2.0 * pairs / nd;
+    cube = 1.0 + 6.0 * (pairs + triples) / nd;
+  } else {
+    mean = std::max(1.0, 2.0 * pairs * nd / (md * md));
+    cube = 6.0 * triples * nd * nd / (md * md * md);
+  }
+  *lanes = knn_cell_lanes(nq, k, mean, cube / (mean * mean));
+  return RTNN_OK;
+}
+
+// Builds the grid of plan_single.  desc_event: separate queries follow, ordered
+// on the second stream as soon as the descriptor is on the device.
+int build_grid(rtnn_ctx ctx, float cell, bool desc_event = true) {
+  GridDesc g;
+  const int rp = plan_single(ctx, cell, g);
+  if (rp) return rp;
   ctx->hgrid = g;
   ctx->ncells = grid_cells(g);
   const uint64_t n = ctx->n;
@@ -915,11 +1009,8 @@ int rtnn_set_points(rtnn_ctx ctx, const float* xyz, uint64_t n, int on_device) {
   if (!xyz) return fail(ctx, RTNN_ERR_INVALID, "xyz is NULL");
   if (n >= 0xffffffffull) return fail(ctx, RTNN_ERR_UNSUPPORTED, "more than 2^32-2 points");
   CK(hipSetDevice(ctx->device));
-  if (!ctx->bbox_tmp.p) {  // the reduction's ticket word, then its partial boxes
-    CK(ctx->bbox_tmp.ensure(256 + kBboxPartBytes));
-    CK(fill_u32(ctx->bbox_tmp.as<uint32_t>(), 1, 0, ctx->st));
-  }
-  CK(ctx->pbbox.ensure(64));
+  const int re = ensure_reduction(ctx);
+  if (re) return re;
   CK(ctx->pts.ensure(12 * n));
   // Points on this device are copied by the kernel that reduces them; others
   // (host memory, another device's) by the runtime before it.
@@ -951,7 +1042,7 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
   if (!qxyz) nq = ctx->n;
   if (nq == 0) return RTNN_OK;
   if (nq >= 0xffffffffull) return fail(ctx, RTNN_ERR_UNSUPPORTED, "more than 2^32-2 queries");
-  const int gl = group_lanes_from_opt(ctx, mode, k);
+  int gl = group_lanes_from_opt(ctx, mode, k);
   const bool pooled = pool_requested(ctx, k);
   if (!pooled && (gl < 0 || k > max_k_for_group(gl))) {
     if (ctx->opt.queries_per_wave > 0 && k <= 1024)
@@ -963,10 +1054,24 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
   const bool timing = wait && (ctx->opt.time_stages != 0 || stats != nullptr);
   if (timing) CK(hipEventRecord(ctx->ev[0], ctx->st));
   // KNN with one query per lane (k <= 64) walks the box tree in packets; queries
-  // left in input order (query_order = 1) make no packets and walk the cells.
-  const bool packet = mode == RTNN_MODE_KNN && gl == 1 && !pooled && ctx->opt.query_order != 1;
+  // left in input order (query_order = 1) make no packets and walk the cells, and
+  // so do, unless one query per lane was asked for, sparse cells (probe_cells).
+  bool packet = mode == RTNN_MODE_KNN && gl == 1 && !pooled && ctx->opt.query_order != 1;
+  bool wide = wide_buffers(ctx);
+  int tiled = tile_points(ctx);
   float f = ctx->opt.cell_factor > 0 ? ctx->opt.cell_factor : default_cell_factor(mode);
   BoxTree tree{};
+  if (packet && wait && ctx->opt.queries_per_wave == 0) {
+    int lanes = 0;
+    rc = probe_cells(ctx, r / f, nq, k, &lanes);
+    if (rc) return rc;
+    if (lanes) {
+      packet = false;
+      gl = lanes;
+      wide = ctx->opt.group_buffer == 2;  // compact buffers serve short lists better
+      tiled = 0;
+    }
+  }
   rc = packet ? build_packet_tree(ctx, &tree) : build_grid(ctx, r / f, qxyz != nullptr);
   if (rc) return rc;
   if (timing) CK(hipEventRecord(ctx->ev[1], ctx->st));
@@ -989,8 +1094,8 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
   if (packet)
     CK(launch_knn_packet(a, tree, ctx->st, ctx->num_cus));
   else
-    CK(launch_search(a, mode == RTNN_MODE_KNN, gl, ctx->st, ctx->num_cus, wide_buffers(ctx),
-                     tile_points(ctx), false, pooled ? ctx->opt.queries_per_wave : 0));
+    CK(launch_search(a, mode == RTNN_MODE_KNN, gl, ctx->st, ctx->num_cus, wide, tiled, false,
+                     pooled ? ctx->opt.queries_per_wave : 0));
   if (timing) CK(hipEventRecord(ctx->ev[3], ctx->st));
   rc = copy_out(ctx, nq, k, out_idx, out_d2, out_on_device, o);
   if (rc) return rc;

@@ -746,6 +746,87 @@ hipError_t cell_count_single(const float* xyz, uint64_t n, const GridDesc& g, Gr
   return hipGetLastError();
 }
 
+// How the points are spread over the cells of grid g, from m of them (all, or
+// draws with replacement): each adds one to its cell's counter, hashed into a
+// table of 2^tbits where that is the smaller, and takes the number of points
+// counted there before it as its rank.  *spread becomes the sums over the draws
+// of rank and of rank (rank - 1) / 2: the pairs and the triples of draws that
+// share a cell.  Random atomics bound it, hence the sample (131,072 draws 10 us,
+// a million points 60); folded by the last block to finish, as in k_bbox.
+__global__ __launch_bounds__(256) void k_cell_spread(const float* __restrict__ xyz, uint64_t n,
+                                                     uint32_t m, const GridDesc g, bool hashed,
+                                                     int tbits, uint32_t* __restrict__ table,
+                                                     unsigned long long* __restrict__ part,
+                                                     uint32_t* __restrict__ ticket,
+                                                     CellSpread* __restrict__ spread) {
+  __shared__ unsigned long long s_sum[2];
+  __shared__ uint32_t s_last;
+  const int lane = threadIdx.x & (kWave - 1);
+  if (threadIdx.x < 2) s_sum[threadIdx.x] = 0;
+  __syncthreads();
+  const uint32_t d = blockIdx.x * 256 + threadIdx.x;
+  const bool valid = d < m;
+  uint32_t key = 0;
+  if (valid) {
+    uint64_t i = d;
+    if (m < n) {  // Steele, Lea and Flood's mixing function (SplitMix64, 2014)
+      uint64_t z = (d + 1ull) * 0x9e3779b97f4a7c15ull;
+      z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+      z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+      i = ((z >> 32) * n) >> 32;
+    }
+    const int cx = cell_of(xyz[3 * i], g.mn[0], g.inv, g.dim[0]);
+    const int cy = cell_of(xyz[3 * i + 1], g.mn[1], g.inv, g.dim[1]);
+    const int cz = cell_of(xyz[3 * i + 2], g.mn[2], g.inv, g.dim[2]);
+    key = ((uint32_t)cz * (uint32_t)g.dim[1] + (uint32_t)cy) * (uint32_t)g.dim[0] + (uint32_t)cx;
+    if (hashed) key = (key * 0x9e3779b1u) >> (32 - tbits);  // Knuth's multiplicative hash
+  }
+  const uint64_t rank = cell_rank(table, key, valid);
+  unsigned long long v[2] = {rank, rank * (rank - (rank ? 1 : 0)) / 2};
+  auto fold = [&]() {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int o = kWave / 2; o > 0; o >>= 1) v[c] += __shfl_xor(v[c], o, kWave);
+      if (lane == 0 && v[c]) atomicAdd(&s_sum[c], v[c]);
+    }
+    __syncthreads();
+  };
+  fold();
+  if (threadIdx.x == 0) {
+    for (int c = 0; c < 2; ++c) {
+      __hip_atomic_store(&part[2 * blockIdx.x + c], s_sum[c], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+      s_sum[c] = 0;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    s_last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+             gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  v[0] = v[1] = 0;
+  for (uint32_t b = threadIdx.x; b < gridDim.x; b += 256)
+    for (int c = 0; c < 2; ++c)
+      v[c] += __hip_atomic_load(&part[2 * b + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  fold();
+  if (threadIdx.x == 0) {
+    spread->pairs = s_sum[0];
+    spread->triples = s_sum[1];
+    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+hipError_t cell_spread(const float* xyz, uint64_t n, uint32_t m, const GridDesc& g, bool hashed,
+                       int tbits, uint32_t* table, uint64_t* part, uint32_t* ticket,
+                       CellSpread* spread, hipStream_t st) {
+  if (m == 0 || m > kSpreadDraws || m > n || tbits < 1 || tbits > 31) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_cell_spread, dim3((m + 255) / 256), dim3(256), 0, st, xyz, n, m, g, hashed,
+                     tbits, table, reinterpret_cast<unsigned long long*>(part), ticket, spread);
+  return hipGetLastError();
+}
+
 hipError_t cell_count(const float* xyz, uint64_t n, const GridDesc* grids,
                       const uint64_t* offsets, uint32_t nclouds, uint32_t* counts, uint32_t* keys,
                       uint32_t* ranks, hipStream_t st) {

@@ -26,6 +26,17 @@ constexpr uint64_t kBboxPartBytes = 4 * 8 * kBboxBlocks;
 // out and nonfinite may be pinned host memory.
 hipError_t bbox(const float* src, float* dst, uint64_t n, float* part, uint32_t* ticket,
                 float* out, uint32_t* nonfinite, hipStream_t st);
+// Pairs and triples of m <= kSpreadDraws points, of n drawn, that share a cell of
+// g.  table: 2^tbits zero words (at least the cells unless hashed), counted up;
+// part: 16 bytes per 256 draws; *ticket: 0 before and after; *spread may be
+// pinned host memory.
+constexpr uint32_t kSpreadDraws = 1u << 17;
+struct CellSpread {
+  uint64_t pairs, triples;
+};
+hipError_t cell_spread(const float* xyz, uint64_t n, uint32_t m, const GridDesc& g, bool hashed,
+                       int tbits, uint32_t* table, uint64_t* part, uint32_t* ticket,
+                       CellSpread* spread, hipStream_t st);
 // Per-cloud bbox: out[6 * c .. 6 * c + 6) for cloud c (offsets: nclouds + 1, n points in all).
 hipError_t bbox_segmented(const float* xyz, const uint64_t* offsets, uint32_t nclouds,
                           uint64_t n, float* out, uint32_t* nonfinite, hipStream_t st);

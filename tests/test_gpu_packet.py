@@ -11,7 +11,9 @@ pytestmark = pytest.mark.gpu
 
 
 def check(ctx, pts, qs, r, k):
+    ctx.set_options(queries_per_wave=64)  # sparse points would go by their cells
     idx, d2, st = ctx.search(qs, mode="knn", radius=r, k=k)
+    ctx.set_options()
     assert st.lanes_per_query == 1
     wi, wd = oracle.grid_search(pts, pts if qs is None else qs, oracle.MODE_KNN, r, k)
     assert np.array_equal(idx, wi) and np.array_equal(d2, wd)
