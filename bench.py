@@ -258,6 +258,8 @@ def kernel_name(res, mode, opts, method):
         return "k_topk_pool"
     if o.get("lds_tile"):
         return "k_topk_tiled"
+    if method == "learned" and res.get("lanes_per_query") == 2:
+        return "k_topk_matrix"
     return "k_topk_group"
 
 

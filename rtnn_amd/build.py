@@ -30,10 +30,11 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall",
 HIP_FLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
              "-packed-fp32-ops", "-fno-gpu-rdc"]
 
-SOURCES = ["sort.hip", "grid.hip", "search.hip", "packet.hip", "partition.hip", "mlp.hip", "api.hip", "data.cpp"]
+SOURCES = ["sort.hip", "grid.hip", "search.hip", "packet.hip", "matrix.hip",
+           "partition.hip", "mlp.hip", "api.hip", "data.cpp"]
 # Per-file flags.  mlp.hip: MFMA results straight into VGPRs (the GELU reads
 # every accumulator; in AGPRs each would first need a v_accvgpr_read).
-EXTRA = {"mlp.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("mlp.hip", "matrix.hip")}
 
 
 def _run(cmd, verbose):

@@ -940,6 +940,7 @@ SearchArgs base_args(rtnn_ctx ctx, const float4* qproc, uint64_t nq, float r, ui
   a.queries = qproc;
   a.tiles = nullptr;
   a.nq = (uint32_t)nq;
+  a.near_pts = qproc == a.spts ? a.nq : ctx->opt.query_order != 1 ? (uint32_t)ctx->n : 0u;
   a.ntiles = (uint32_t)((nq + kTileQ - 1) / kTileQ);
   a.r = r;
   a.qradius_scale = 1.0f;
@@ -3056,6 +3057,7 @@ hipError_t enqueue_batched(rtnn_graph g, const float* xyz, float cell, int mode,
   a.tiles = g->tiles.as<Tile>();
   a.ntiles = g->ntiles;
   a.nq = (uint32_t)g->n;
+  a.near_pts = a.nq;
   a.r = r;
   a.qradius_scale = 1.0f;
   a.k = k;

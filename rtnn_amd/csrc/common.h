@@ -51,6 +51,8 @@ struct SearchArgs {
   uint32_t tile_q;           // queries per implicit tile (set by launch_search)
   uint32_t ntiles;
   uint32_t nq;
+  uint32_t near_pts;         // points searched, where consecutive queries are
+                             // neighbours (in cell or curve order); 0: not so
   float r;                   // search radius (per-query radius overrides when set)
   uint32_t k;                // output columns
   const float* qradius;      // nullable; indexed by processing position (queries[])

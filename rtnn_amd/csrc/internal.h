@@ -137,6 +137,11 @@ hipError_t bucket_snap(float* qradius, uint32_t nq, float snap_r, float r, hipSt
 hipError_t launch_search(const SearchArgs& a, int knn_mode, int group_lanes, hipStream_t st,
                          int num_cus, bool wide = true, int tiled = 0, bool deep = false,
                          int pool = 0);
+// ---- matrix.hip
+// Range search or KNN (k <= 32) over raster grids by 64 queries per wave, the
+// distances filtered on the matrix cores (one block per tile; no device-resident
+// query count).  launch_search chooses it.
+hipError_t launch_matrix(const SearchArgs& a, bool knn, hipStream_t st);
 // ---- packet.hip
 // Level layout of the box tree of n points over `box` (2 * boxes float4).
 BoxTree box_tree_layout(uint64_t n, float4* box);

@@ -169,23 +169,6 @@ __device__ inline const_f4 uniform_ptr(const float4* p, uint32_t i) {
   return (const_f4)(p + (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)i));
 }
 
-// Lane moves that leave the identity of an unsigned minimum where no lane is
-// read, so that each folds into its v_min_u32.
-template <int CTRL, int ROWS>
-__device__ inline uint32_t dpp_or_max(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, CTRL, ROWS, 0xf, false);
-}
-// Minimum over the wave, uniform (row shifts, then the two row broadcasts).
-__device__ inline uint32_t wave_min_u32(uint32_t v) {
-  v = min(v, dpp_or_max<0x111, 0xf>(v));
-  v = min(v, dpp_or_max<0x112, 0xf>(v));
-  v = min(v, dpp_or_max<0x114, 0xf>(v));
-  v = min(v, dpp_or_max<0x118, 0xf>(v));
-  v = min(v, dpp_or_max<0x142, 0xa>(v));
-  v = min(v, dpp_or_max<0x143, 0xc>(v));
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, kWave - 1);
-}
-__device__ inline uint32_t wave_max_u32(uint32_t v) { return ~wave_min_u32(~v); }
 __device__ inline float wave_min_f(float v) {
 #pragma unroll
   for (int o = kWave / 2; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, kWave));

@@ -33,48 +33,6 @@
 
 namespace rtnn {
 
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Resolves tile t into its query range and grid.
-__device__ inline void tile_of(const SearchArgs& a, uint32_t nq, uint32_t t, uint32_t& q0,
-                               uint32_t& q1, uint32_t& gi) {
-  if (a.tiles) {
-    Tile tl = a.tiles[t];
-    q0 = tl.q0; q1 = tl.q1; gi = tl.grid;
-  } else {
-    q0 = t * a.tile_q;
-    q1 = min(q0 + a.tile_q, nq);
-    gi = 0;
-  }
-}
-
-// Persistent launches walk tiles in XCD-contiguous chunks; plain launches map
-// each block to one tile through xcd_swizzle.
-struct TileIter {
-  uint32_t t, end, step;
-  __device__ TileIter(const SearchArgs& a, uint32_t nq) {
-    uint32_t ntiles = a.nq_dev ? (nq + a.tile_q - 1) / a.tile_q : a.ntiles;
-    if (a.persistent) {
-      constexpr uint32_t kXcd = 8;
-      uint32_t x = blockIdx.x % kXcd, j = blockIdx.x / kXcd;
-      uint32_t per = (gridDim.x + kXcd - 1 - x) / kXcd;  // blocks on this XCD
-      uint32_t q = ntiles / kXcd, rem = ntiles % kXcd;
-      uint32_t start = x * q + (x < rem ? x : rem);
-      end = start + q + (x < rem ? 1u : 0u);
-      t = start + j;
-      step = per;
-    } else {
-      t = xcd_swizzle(blockIdx.x, gridDim.x);
-      end = t + 1;
-      step = 1;
-    }
-  }
-};
-
 // Candidates loaded per lane before the first is tested (thread kernel;
 // group kernel: its G lanes share a query, so each lane takes more), and
 // runs (rows or cells) whose bounds each group lane loads per batch.
@@ -1197,6 +1155,25 @@ uint32_t max_k_for_group(int group_lanes) {
   }
 }
 
+// Whether the matrix kernel takes the place of the group kernel: range searches
+// at the default 16 lanes per query and KNN at proposed radii with 2, up to the
+// keys its registers hold.  A wave takes 64 queries, so it wants many of them
+// (graph-captured batches excepted: the group kernel walks those 256 queries at a
+// time) that are neighbours and not much sparser than the points.  Pass time,
+// group / matrix kernel, us: uniform points, r = 2.4, K = 32: 100k 137 / 152,
+// 300k 296 / 206, 1M 855 / 437; r = 1.2 (6 hits a query), K = 8: 300k 170 / 179,
+// 1M 429 / 352; sphere surfaces, K = 32: 1.2M points and 0.3M queries 345 / 409,
+// 2M and 2M 1269 / 804, K = 8 1482 / 746.  Batches of lattices, K = 32: 8 clouds
+// (18k points) 152 / 93, 48 167 / 112, 200 341 / 216.  (At 4 lanes and compact
+// buffers, which a tuned program sets, the group kernel is 1.1 times as fast.)
+static bool matrix_rule(const SearchArgs& a, bool knn, int group_lanes, int tiled) {
+  if (a.nlevels > 0 || tiled != 0 || a.nq_dev || a.qsel || a.near_pts == 0) return false;
+  if (knn ? !a.qradius || group_lanes != 2 || a.k > 16 || a.tiles
+          : group_lanes != 16 || a.k > 32)
+    return false;
+  return a.tiles || (a.nq >= 1u << 19 && a.nq >= a.near_pts / 2);
+}
+
 hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hipStream_t st,
                          int num_cus, bool wide, int tiled, bool deep, int pool) {
   SearchArgs a = a0;
@@ -1234,6 +1211,8 @@ hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hi
     return launch_search(o, knn_mode, 4, st, num_cus, true, 0, true, 0);
   }
   if (k == 0 || k > max_k_for_group(group_lanes)) return hipErrorInvalidValue;
+  if (matrix_rule(a, knn_mode != 0, group_lanes, tiled))
+    return launch_matrix(a, knn_mode != 0, st);
   // hierarchical grids: KNN by groups (one lane per query is the packet walk's)
   if (a.nlevels > 0 && (group_lanes == 1 || !knn_mode)) return hipErrorInvalidValue;
   if (!a.tiles) {

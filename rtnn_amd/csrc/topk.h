@@ -1,5 +1,5 @@
-// Device helpers of the top-k kernels: keys as doubles, query radius, the
-// short-row list.
+// Device helpers of the top-k kernels: query tiles, wave reductions, keys as
+// doubles, query radius, the short-row list.
 #pragma once
 
 #include "common.h"
@@ -50,6 +50,68 @@ __device__ inline float query_radius(const SearchArgs& a, uint32_t qi, uint32_t 
   return fminf(a.r, a.qradius[qs] * sc);
 }
 
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Resolves tile t into its query range and grid.
+__device__ __forceinline__ void tile_of(const SearchArgs& a, uint32_t nq, uint32_t t, uint32_t& q0,
+                               uint32_t& q1, uint32_t& gi) {
+  if (a.tiles) {
+    Tile tl = a.tiles[t];
+    q0 = tl.q0; q1 = tl.q1; gi = tl.grid;
+  } else {
+    q0 = t * a.tile_q;
+    q1 = min(q0 + a.tile_q, nq);
+    gi = 0;
+  }
+}
+
+// Persistent launches walk tiles in XCD-contiguous chunks; plain launches map
+// each block to one tile through xcd_swizzle.
+struct TileIter {
+  uint32_t t, end, step;
+  __device__ __forceinline__ TileIter(const SearchArgs& a, uint32_t nq) {
+    uint32_t ntiles = a.nq_dev ? (nq + a.tile_q - 1) / a.tile_q : a.ntiles;
+    if (a.persistent) {
+      constexpr uint32_t kXcd = 8;
+      uint32_t x = blockIdx.x % kXcd, j = blockIdx.x / kXcd;
+      uint32_t per = (gridDim.x + kXcd - 1 - x) / kXcd;  // blocks on this XCD
+      uint32_t q = ntiles / kXcd, rem = ntiles % kXcd;
+      uint32_t start = x * q + (x < rem ? x : rem);
+      end = start + q + (x < rem ? 1u : 0u);
+      t = start + j;
+      step = per;
+    } else {
+      t = xcd_swizzle(blockIdx.x, gridDim.x);
+      end = t + 1;
+      step = 1;
+    }
+  }
+};
+
+// ---- wave reductions
+
+// Lane moves that leave the identity of an unsigned minimum where no lane is
+// read, so that each folds into its v_min_u32.
+template <int CTRL, int ROWS>
+__device__ inline uint32_t dpp_or_max(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, CTRL, ROWS, 0xf, false);
+}
+// Minimum over the wave, uniform (row shifts, then the two row broadcasts).
+__device__ inline uint32_t wave_min_u32(uint32_t v) {
+  v = min(v, dpp_or_max<0x111, 0xf>(v));
+  v = min(v, dpp_or_max<0x112, 0xf>(v));
+  v = min(v, dpp_or_max<0x114, 0xf>(v));
+  v = min(v, dpp_or_max<0x118, 0xf>(v));
+  v = min(v, dpp_or_max<0x142, 0xa>(v));
+  v = min(v, dpp_or_max<0x143, 0xc>(v));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, kWave - 1);
+}
+__device__ inline uint32_t wave_max_u32(uint32_t v) { return ~wave_min_u32(~v); }
+
 // ---- keys as doubles
 //
 // A key (d2 bits << 32 | index) of a finite d2 >= 0 is the bit pattern of a
@@ -77,12 +139,21 @@ __device__ inline void key_cx(double& a, double& b) {
   a = lo;
 }
 
+// The same with a and b in the registers they are in, for a list that lives
+// across a loop: with key_cx its keys change registers, and the copies back at
+// the loop's joins were spilled.
+__device__ inline void key_cx_inplace(double& a, double& b) {
+  double lo;
+  asm volatile("v_min_f64 %0, %1, %2\n\tv_max_f64 %2, %1, %2\n\tv_mov_b64 %1, %0"
+               : "=&v"(lo), "+v"(a), "+v"(b));
+}
+
 // Sorts N keys ascending: Batcher's odd-even merge sort of the next power of
 // two, whose missing last keys would be the largest (12 keys: 41
 // compare-exchanges).  One comparator level per template instance,
 // so that every index is a constant and the keys stay in registers.
 template <int N, int P, int Q>
-__device__ inline void sort_level(double (&v)[N]) {
+__device__ __forceinline__ void sort_level(double (&v)[N]) {
 #pragma unroll
   for (int i = 0; i < N - Q; ++i) {
     const int off = i - Q % P;
@@ -94,12 +165,12 @@ __device__ inline void sort_level(double (&v)[N]) {
     sort_level<N, 2 * P, 2 * P>(v);
 }
 template <int N>
-__device__ inline void sort_keys(double (&v)[N]) {
+__device__ __forceinline__ void sort_keys(double (&v)[N]) {
   sort_level<N, 1, 1>(v);
 }
 
 template <int KC, int H>
-__device__ inline void bitonic_level(double (&list)[KC]) {
+__device__ __forceinline__ void bitonic_level(double (&list)[KC]) {
 #pragma unroll
   for (int i = 0; i < KC; ++i)
     if ((i & H) == 0) key_cx(list[i], list[i + H]);
@@ -110,11 +181,27 @@ __device__ inline void bitonic_level(double (&list)[KC]) {
 // last keys against v reversed leaves a bitonic sequence of the smallest,
 // which a bitonic merge orders.
 template <int KC, int NB>
-__device__ inline void merge_keys(double (&list)[KC], const double (&v)[NB]) {
+__device__ __forceinline__ void merge_keys(double (&list)[KC], const double (&v)[NB]) {
 #pragma unroll
   for (int i = 0; i < (KC < NB ? KC : NB); ++i)
     list[KC - 1 - i] = key_min(list[KC - 1 - i], v[i]);
   bitonic_level<KC, KC / 2>(list);
+}
+
+// The same on a list that keeps its registers.
+template <int KC, int H>
+__device__ __forceinline__ void bitonic_level_inplace(double (&list)[KC]) {
+#pragma unroll
+  for (int i = 0; i < KC; ++i)
+    if ((i & H) == 0) key_cx_inplace(list[i], list[i + H]);
+  if constexpr (H > 1) bitonic_level_inplace<KC, H / 2>(list);
+}
+template <int KC, int NB>
+__device__ __forceinline__ void merge_keys_inplace(double (&list)[KC], const double (&v)[NB]) {
+#pragma unroll
+  for (int i = 0; i < (KC < NB ? KC : NB); ++i)
+    asm volatile("v_min_f64 %0, %0, %1" : "+v"(list[KC - 1 - i]) : "v"(v[i]));
+  bitonic_level_inplace<KC, KC / 2>(list);
 }
 
 }  // namespace rtnn
