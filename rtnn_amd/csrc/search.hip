@@ -1156,21 +1156,22 @@ uint32_t max_k_for_group(int group_lanes) {
 }
 
 // Whether the matrix kernel takes the place of the group kernel: range searches
-// at the default 16 lanes per query and KNN at proposed radii with 2, up to the
-// keys its registers hold.  A wave takes 64 queries, so it wants many of them
+// at the default 16 lanes per query, KNN at proposed radii with 2 and in batches
+// with one, up to the keys its registers hold.  A wave takes 64 queries, so it wants many of them
 // (graph-captured batches excepted: the group kernel walks those 256 queries at a
 // time) that are neighbours and not much sparser than the points.  Pass time,
 // group / matrix kernel, us: uniform points, r = 2.4, K = 32: 100k 137 / 152,
 // 300k 296 / 206, 1M 855 / 437; r = 1.2 (6 hits a query), K = 8: 300k 170 / 179,
 // 1M 429 / 352; sphere surfaces, K = 32: 1.2M points and 0.3M queries 345 / 409,
 // 2M and 2M 1269 / 804, K = 8 1482 / 746.  Batches of lattices, K = 32: 8 clouds
-// (18k points) 152 / 93, 48 167 / 112, 200 341 / 216.  (At 4 lanes and compact
+// (18k points) 152 / 93, 48 167 / 112, 200 341 / 216; KNN of 200, one lane each
+// against it: K = 16 357 / 207, r = 0.3 and K = 32 1443 / 388.  (At 4 lanes and compact
 // buffers, which a tuned program sets, the group kernel is 1.1 times as fast.)
 static bool matrix_rule(const SearchArgs& a, bool knn, int group_lanes, int tiled) {
   if (a.nlevels > 0 || tiled != 0 || a.nq_dev || a.qsel || a.near_pts == 0) return false;
-  if (knn ? !a.qradius || group_lanes != 2 || a.k > 16 || a.tiles
-          : group_lanes != 16 || a.k > 32)
-    return false;
+  if (!knn && (group_lanes != 16 || a.k > 32)) return false;
+  if (knn && a.tiles && (group_lanes != 1 || a.k > 32)) return false;
+  if (knn && !a.tiles && (!a.qradius || group_lanes != 2 || a.k > 16)) return false;
   return a.tiles || (a.nq >= 1u << 19 && a.nq >= a.near_pts / 2);
 }
 
@@ -1213,6 +1214,13 @@ hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hi
   if (k == 0 || k > max_k_for_group(group_lanes)) return hipErrorInvalidValue;
   if (matrix_rule(a, knn_mode != 0, group_lanes, tiled))
     return launch_matrix(a, knn_mode != 0, st);
+  // KNN of longer rows in batches: 16 lanes each, where one lane each inserts
+  // every hit of its wave one by one (200 lattices, K = 48: 358 us against
+  // 2272; with r = 0.6, far more hits than K, 3.7 ms against 14.9).
+  if (knn_mode && a.tiles && group_lanes == 1 && k > 32 && a.nlevels == 0) {
+    group_lanes = 16;
+    tiled = 0;
+  }
   // hierarchical grids: KNN by groups (one lane per query is the packet walk's)
   if (a.nlevels > 0 && (group_lanes == 1 || !knn_mode)) return hipErrorInvalidValue;
   if (!a.tiles) {

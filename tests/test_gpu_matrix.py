@@ -64,6 +64,7 @@ def test_batches(ctx, k, scale, r):
     xyz = (rng.uniform(0, 1, (int(offs[-1]), 3)) * scale).astype(np.float32)
     dev = torch.from_numpy(xyz).cuda()
     torch.cuda.synchronize()
+    ctx.set_options()
     idx, d2, _ = ctx.search_batched(dev, offs, radius=r, k=k)
     idx, d2 = idx.cpu().numpy(), d2.cpu().numpy()
     for a, b in zip(offs[:-1].astype(int), offs[1:].astype(int)):
@@ -83,4 +84,23 @@ def test_knn_at_proposed_radii(ctx, k):
     want = ctx.search(pts, mode="knn", radius=4.0, k=k)
     ctx.set_options(cell_factor=2.0, queries_per_wave=32, grid_levels=1, group_buffer=2)
     got = ctx.search_learned(pts, radius=4.0, k=k)
+    ctx.set_options()
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("k", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("r", [0.2, 0.5, 5.0])
+def test_knn_batches(ctx, k, r):
+    rng = np.random.default_rng(9)
+    sizes = [1, 2, 31, 33, 64, 65, 255, 257, 769, 1500]
+    offs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
+    xyz = rng.uniform(0, 1, (int(offs[-1]), 3)).astype(np.float32)
+    xyz[-40:] = xyz[-1]  # duplicates are no neighbours of each other
+    dev = torch.from_numpy(xyz).cuda()
+    torch.cuda.synchronize()
+    ctx.set_options()
+    idx, d2, _ = ctx.search_batched(dev, offs, mode="knn", radius=r, k=k)
+    idx, d2 = idx.cpu().numpy(), d2.cpu().numpy()
+    for a, b in zip(offs[:-1].astype(int), offs[1:].astype(int)):
+        wi, wd = oracle.bruteforce(xyz[a:b], xyz[a:b], oracle.MODE_KNN, r, k)
+        assert np.array_equal(idx[a:b], wi) and np.array_equal(d2[a:b], wd)
