@@ -18,14 +18,14 @@
 // batches are sorted and merged into the row in registers, all lanes at once
 // (v_min_f64 / v_max_f64, see topk.h).
 //
-// A wave's latency bounds it at 8 waves per CU, which the 20 KB of LDS per wave
-// allow: the products take a fifth of it, the loads of the block and the stores
+// A wave's latency bounds it at the 12 (K <= 16) or 8 waves per CU that its LDS
+// allows: the products take a fifth of it, the loads of the block and the stores
 // of the rows most of the rest.  Rows of 64 keys would need every register there
 // is and spill (batches of 1024 clouds, K = 64: 20 ms against the group kernel's
 // 13.6), so k > 32 stays with the groups.  A pass against groups of lanes per
 // query, which test each query's candidates alone: 1M uniform points, r = 2.4,
-// K = 32: 855 -> 437 us; 2M queries on sphere surfaces, K = 8: 1482 -> 746 us;
-// learned KNN of 10M, K = 16: 5.23 -> 4.32 ms; 48 small clouds 167 -> 112 us.
+// K = 32: 855 -> 437 us; 2M queries on sphere surfaces, K = 8: 1482 -> 686 us;
+// learned KNN of 10M, K = 16: 5.23 -> 3.99 ms; 48 small clouds 167 -> 112 us.
 #include <float.h>
 
 #include <algorithm>
@@ -46,10 +46,17 @@ constexpr int kMatTile = 32;   // points per product
 // many of the first one's: x is free along a row of cells (the block holds only
 // the points there are), y and z multiply the rows.
 constexpr int kSpanX = 16, kSpanYZ = 4;
-constexpr int kTiles = 24;     // tiles listed before their hits are taken
 constexpr int kBatch = 16;     // keys sorted at a time
 constexpr int kStep = 8;       // of them read at a time
-constexpr uint32_t kCap = kTiles * kMatTile;
+
+// Tiles listed before their hits are taken, and the waves per SIMD that their LDS
+// and the row's registers leave.  K <= 16 has registers for three: 15 tiles make
+// room for them (learned KNN of 10M 4.31 -> 3.99 ms against 24 and two).
+template <int KC>
+struct MatCfg {
+  static constexpr int kTiles = KC <= 16 ? 15 : 24;
+  static constexpr int kOccupancy = KC <= 16 ? 3 : 2;
+};
 
 // No key: what an empty slot of a row holds, d2 = inf and index -1.  Above every
 // key, and as a double still finite.
@@ -100,7 +107,10 @@ __device__ __forceinline__ void emit_row(const SearchArgs& a, const double (&lis
 
 template <int KC, bool KNN>
 __global__ __launch_bounds__(kTileQ)
-__attribute__((amdgpu_waves_per_eu(2))) void k_topk_matrix(const SearchArgs a) {
+__attribute__((amdgpu_waves_per_eu(MatCfg<KC>::kOccupancy))) void k_topk_matrix(
+    const SearchArgs a) {
+  constexpr int kTiles = MatCfg<KC>::kTiles;
+  constexpr uint32_t kCap = kTiles * kMatTile;
   __shared__ float4 s_pts[kMatWaves][kCap];                  // listed points
   __shared__ uint32_t s_word[kMatWaves][kTiles + 1][kWave];  // a lane's non-zero words, then 0
   __shared__ uint8_t s_tile[kMatWaves][kTiles + 1][kWave];   // and their tiles

@@ -1162,8 +1162,8 @@ uint32_t max_k_for_group(int group_lanes) {
 // time) that are neighbours and not much sparser than the points.  Pass time,
 // group / matrix kernel, us: uniform points, r = 2.4, K = 32: 100k 137 / 152,
 // 300k 296 / 206, 1M 855 / 437; r = 1.2 (6 hits a query), K = 8: 300k 170 / 179,
-// 1M 429 / 352; sphere surfaces, K = 32: 1.2M points and 0.3M queries 345 / 409,
-// 2M and 2M 1269 / 804, K = 8 1482 / 746.  Batches of lattices, K = 32: 8 clouds
+// 1M 429 / 320; sphere surfaces, K = 32: 1.2M points and 0.3M queries 345 / 409,
+// 2M and 2M 1269 / 804, K = 8 1482 / 686.  Batches of lattices, K = 32: 8 clouds
 // (18k points) 152 / 93, 48 167 / 112, 200 341 / 216; KNN of 200, one lane each
 // against it: K = 16 357 / 207, r = 0.3 and K = 32 1443 / 388.  (At 4 lanes and compact
 // buffers, which a tuned program sets, the group kernel is 1.1 times as fast.)
