@@ -176,6 +176,36 @@ struct PinBuf {
 constexpr size_t kScratchBytes = 128ull << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
+namespace rtnn {
+NoallocLayout noalloc_layout(uint64_t n, uint64_t nq, bool own_q, bool pooled) {
+  uint64_t used = 0;
+  auto take = [&](uint64_t bytes) {
+    const uint64_t at = used;
+    used += (bytes + 255) & ~255ull;
+    return at;
+  };
+  const uint64_t sort_words = std::max(radix_tmp_words(n), own_q ? radix_tmp_words(nq) : 0);
+  NoallocLayout l{};
+  l.status = take(16);
+  l.offs = take(16);
+  l.bb = take(4 * 6);
+  l.grid = take(sizeof(GridDesc));
+  l.keys = take(4 * n);
+  l.vals = take(4 * n);
+  l.spts = take(16 * n + kSptsPadBytes);
+  l.tmp = take(std::max({4 * sort_words, 4 * cell_bounds_tmp_words(kScratchBytes / 4),
+                         kBboxPartBytes}));
+  if (own_q) {
+    l.qkeys = take(4 * nq);
+    l.qvals = take(4 * nq);
+    l.qs = take(16 * nq);
+  }
+  if (pooled) l.ovf = take(4 * (nq + 64));
+  l.cells = used;
+  return l;
+}
+}  // namespace rtnn
+
 namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -1309,25 +1339,9 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
                     "hipGetSymbolAddress(scratch)");
   // Carve the scratch (256-byte aligned pieces); sizes beyond it are refused.
   const bool own_q = qxyz != nullptr;
-  const uint64_t sort_n = std::max(n, own_q ? nq : 0);
-  uint64_t used = 0;
-  auto take = [&](uint64_t bytes) -> uint64_t {
-    const uint64_t at = used;
-    used += (bytes + 255) & ~255ull;
-    return at;
-  };
-  const uint64_t o_status = take(16), o_offs = take(16), o_part = take(kBboxPartBytes);
-  const uint64_t o_bb = take(4 * 6), o_grid = take(sizeof(GridDesc));
-  const uint64_t o_keys = take(4 * n), o_vals = take(4 * n);
-  const uint64_t o_spts = take(16 * n + kSptsPadBytes);
-  const uint64_t o_tmp = take(4 * std::max(radix_tmp_words(sort_n),
-                                           cell_bounds_tmp_words(kScratchBytes / 4)));
-  const uint64_t o_qkeys = own_q ? take(4 * nq) : 0, o_qvals = own_q ? take(4 * nq) : 0;
-  const uint64_t o_qs = own_q ? take(16 * nq) : 0;
-  const uint64_t o_ovf = pooled ? take(4 * (nq + 64)) : 0;
-  const uint64_t o_cells = take(0);
+  const NoallocLayout at = noalloc_layout(n, nq, own_q, pooled);
   constexpr uint64_t kMinCells = 1ull << 16;
-  if (o_cells + 4 * (kMinCells + 1) > kScratchBytes)
+  if (at.cells + 4 * (kMinCells + 1) > kScratchBytes)
     return fail(ctx, RTNN_ERR_UNSUPPORTED,
                 "%llu points and %llu queries exceed the %llu MiB scratch of "
                 "rtnn_search_noalloc (about 40 B per point, 24 B per separate query, and "
@@ -1335,19 +1349,19 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
                 (unsigned long long)n, (unsigned long long)(own_q ? nq : 0),
                 (unsigned long long)(kScratchBytes >> 20));
   // The cell table takes the rest, up to the cell budget of rtnn_search.
-  const uint64_t cap = std::min<uint64_t>(std::min<uint64_t>((kScratchBytes - o_cells) / 4 - 1,
+  const uint64_t cap = std::min<uint64_t>(std::min<uint64_t>((kScratchBytes - at.cells) / 4 - 1,
                                                              max_cells_for(ctx, n)),
                                           0xfffffff0ull);
   unsigned char* base = static_cast<unsigned char*>(ctx->scratch);
-  uint32_t* status = reinterpret_cast<uint32_t*>(base + o_status);
-  uint64_t* offs = reinterpret_cast<uint64_t*>(base + o_offs);
-  float* bb = reinterpret_cast<float*>(base + o_bb);
-  GridDesc* grid = reinterpret_cast<GridDesc*>(base + o_grid);
-  uint32_t* keys = reinterpret_cast<uint32_t*>(base + o_keys);
-  uint32_t* vals = reinterpret_cast<uint32_t*>(base + o_vals);
-  float4* spts = reinterpret_cast<float4*>(base + o_spts);
-  uint32_t* tmp = reinterpret_cast<uint32_t*>(base + o_tmp);
-  uint32_t* cell_start = reinterpret_cast<uint32_t*>(base + o_cells);
+  uint32_t* status = reinterpret_cast<uint32_t*>(base + at.status);
+  uint64_t* offs = reinterpret_cast<uint64_t*>(base + at.offs);
+  float* bb = reinterpret_cast<float*>(base + at.bb);
+  GridDesc* grid = reinterpret_cast<GridDesc*>(base + at.grid);
+  uint32_t* keys = reinterpret_cast<uint32_t*>(base + at.keys);
+  uint32_t* vals = reinterpret_cast<uint32_t*>(base + at.vals);
+  float4* spts = reinterpret_cast<float4*>(base + at.spts);
+  uint32_t* tmp = reinterpret_cast<uint32_t*>(base + at.tmp);
+  uint32_t* cell_start = reinterpret_cast<uint32_t*>(base + at.cells);
   CK(hipSetDevice(ctx->device));
   hipStream_t st = ctx->st;
   // status: [0] non-finite coordinates, [1] planning fell back, [2] cells,
@@ -1356,8 +1370,7 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
   CK(fill_u32(status, 4, 0, st));
   CK(fill_u32(reinterpret_cast<uint32_t*>(offs), 4, 0, st));
   CK(fill_u32(reinterpret_cast<uint32_t*>(offs) + 2, 1, (uint32_t)n, st));
-  CK(bbox(xyz, nullptr, n, reinterpret_cast<float*>(base + o_part), &status[3], bb, &status[0],
-          st));
+  CK(bbox(xyz, nullptr, n, reinterpret_cast<float*>(tmp), &status[3], bb, &status[0], st));
   const float f = ctx->opt.cell_factor > 0 ? ctx->opt.cell_factor : default_cell_factor(mode);
   CK(plan_batched(bb, offs, 1, r / f, nullptr, cap, grid, status, st));
   CK(cell_keys(xyz, n, grid, offs, 1, keys, vals, nullptr, st));
@@ -1366,9 +1379,9 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
   CK(gather_points(xyz, vals, n, spts, st));
   const float4* qproc = spts;
   if (own_q) {
-    uint32_t* qkeys = reinterpret_cast<uint32_t*>(base + o_qkeys);
-    uint32_t* qvals = reinterpret_cast<uint32_t*>(base + o_qvals);
-    float4* qs = reinterpret_cast<float4*>(base + o_qs);
+    uint32_t* qkeys = reinterpret_cast<uint32_t*>(base + at.qkeys);
+    uint32_t* qvals = reinterpret_cast<uint32_t*>(base + at.qvals);
+    float4* qs = reinterpret_cast<float4*>(base + at.qs);
     if (ctx->opt.query_order == 1) {
       CK(iota_u32(qvals, nq, st));
     } else {
@@ -1391,7 +1404,7 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
   a.out_idx = out_idx;
   a.out_d2 = out_d2;
   if (pooled) {
-    a.ovf_count = reinterpret_cast<uint32_t*>(base + o_ovf);
+    a.ovf_count = reinterpret_cast<uint32_t*>(base + at.ovf);
     a.ovf_rows = a.ovf_count + 64;
     CK(fill_u32(a.ovf_count, 1, 0, st));
   }

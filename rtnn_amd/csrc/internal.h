@@ -14,6 +14,9 @@ namespace rtnn {
 int scan_tmp_words(uint64_t n);
 hipError_t exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp,
                           hipStream_t st);
+// Words of tmp that radix_sort_pairs of n pairs writes.  Not monotone in n (the
+// tile size changes at half a million): a workspace of several sorts takes the
+// largest of their own words.
 uint64_t radix_tmp_words(uint64_t n);
 hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint64_t n, int bits,
                             uint32_t* tmp, hipStream_t st, int* passes_out);
@@ -151,6 +154,17 @@ hipError_t build_box_tree(const float* xyz, const uint32_t* vals, uint64_t n, fl
                           const BoxTree& t, hipStream_t st);
 // KNN (k <= 64) of a's queries over the box tree of a.spts.
 hipError_t launch_knn_packet(const SearchArgs& a, const BoxTree& t, hipStream_t st, int num_cus);
+
+// ---- api.hip
+// Scratch of rtnn_search_noalloc: byte offsets of its pieces, 256-byte aligned
+// and in this order (a piece ends where the next one used starts; qkeys, qvals
+// and qs with separate queries only, ovf for the pooled kernel only, the cell
+// table last).  tmp serves the box reduction, then both sorts and the cell table,
+// one after the other.
+struct NoallocLayout {
+  uint64_t status, offs, bb, grid, keys, vals, spts, tmp, qkeys, qvals, qs, ovf, cells;
+};
+NoallocLayout noalloc_layout(uint64_t n, uint64_t nq, bool own_q, bool pooled);
 
 // Every device / pinned allocation of the library (tracked for
 // rtnn_mem_stats; logged with RTNN_MEMSTAT set).
