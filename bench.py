@@ -247,7 +247,10 @@ def proposal_tune(ctx, dq, r, k, spec, base_opts):
 def kernel_name(res, mode, opts, method):
     """Name of the dominant search kernel of a method's configuration."""
     o = opts or {}
+    qpw = o.get("queries_per_wave", 0)
     if res.get("lanes_per_query") == 1 and not o.get("group_buffer") == 3:
+        if 0 < qpw < 64 or (qpw == 0 and mode != "knn"):  # groups were asked for
+            return "k_topk_matrix"
         if mode == "knn" and method == "plain" and list(res.get("grid_dims", ())) != [1024] * 3:
             return "k_topk_thread"
         if mode == "knn" and (method == "plain" or o.get("grid_levels", 0) >= 2 or
@@ -258,8 +261,6 @@ def kernel_name(res, mode, opts, method):
         return "k_topk_pool"
     if o.get("lds_tile"):
         return "k_topk_tiled"
-    if method == "learned" and res.get("lanes_per_query") == 2:
-        return "k_topk_matrix"
     return "k_topk_group"
 
 

@@ -111,7 +111,8 @@ typedef struct {
   float    cell_size;
   uint32_t sort_passes;   /* LSD radix passes of the point sort (0: counted into cells) */
   uint32_t search_launches;
-  uint32_t lanes_per_query; /* range kernel group width actually used               */
+  uint32_t lanes_per_query; /* lanes per query of the (first) search kernel that ran;
+                               1: one query per lane                               */
   double ms_copy;         /* result copy to host arrays (host outputs only)          */
 } rtnn_stats;
 

@@ -1278,7 +1278,9 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
     stats->ms_copy = out_on_device ? 0.0 : ev_ms(ctx->ev[3], ev_copied);
     stats->ms_total = ev_ms(ctx->ev[0], ev_copied);
     stats->search_launches = pooled ? 2 : 1;
-    stats->lanes_per_query = pooled ? (uint32_t)(64 / ctx->opt.queries_per_wave) : (uint32_t)gl;
+    stats->lanes_per_query = (uint32_t)(pooled   ? 64 / ctx->opt.queries_per_wave
+                                        : packet ? 1
+                                                 : lanes_used(a, mode == RTNN_MODE_KNN, gl, tiled));
     fill_stats(ctx, stats);
   }
   return RTNN_OK;
@@ -1681,7 +1683,9 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
     stats->ms_total = ev_ms(ctx->ev[0], ctx->ev[5]);
     stats->fallback_queries = nshort;
     stats->search_launches = 2 + (tree_fallback ? 0 : kGrowStages) + (pooled ? 1 : 0);
-    stats->lanes_per_query = pooled ? (uint32_t)(64 / ctx->opt.queries_per_wave) : (uint32_t)gl;
+    stats->lanes_per_query = (uint32_t)(pooled            ? 64 / ctx->opt.queries_per_wave
+                                        : walk && gl == 1 ? 1
+                                                          : lanes_used(a, true, gl, tile_points(ctx)));
     fill_stats(ctx, stats);
   }
   return RTNN_OK;
@@ -2325,6 +2329,14 @@ int opt_lanes(const rtnn_options& o, int mode, uint32_t k) {
   return qpw > 0 ? 64 / qpw : default_group_lanes(mode, k);
 }
 
+// A batch of one cloud: implicit tiles over all its points.
+SearchArgs one_cloud_args(SearchArgs a) {
+  a.tiles = nullptr;
+  a.ntiles = 0;
+  a.persistent = 0;
+  return a;
+}
+
 // The batched search over a's tiles: one persistent launch with options o, or
 // with size classes one per class over its tile range with its options.
 hipError_t launch_batched(const SearchArgs& a, int mode, uint32_t k, int num_cus,
@@ -2336,11 +2348,7 @@ hipError_t launch_batched(const SearchArgs& a, int mode, uint32_t k, int num_cus
     // One cloud: the plain launch (implicit tiles over all its points, as
     // many blocks as the queries fill) instead of the persistent walk of the
     // batch's 256-query tile list, which leaves CUs idle on small batches.
-    SearchArgs b = a;
-    b.tiles = nullptr;
-    b.ntiles = 0;
-    b.persistent = 0;
-    return launch_search(b, knn, opt_lanes(o, mode, k), st, num_cus, o.group_buffer != 1,
+    return launch_search(one_cloud_args(a), knn, opt_lanes(o, mode, k), st, num_cus, o.group_buffer != 1,
                          o.lds_tile == 1 ? 512 : o.lds_tile);
   }
   if (copt.empty())
@@ -2523,7 +2531,10 @@ int batched_impl(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets, uint32
     stats->ms_search = ev_ms(ctx->ev[1], ctx->ev[2]);
     stats->ms_total = ev_ms(ctx->ev[0], ctx->ev[2]);
     stats->search_launches = (uint32_t)std::max<size_t>(1, ctx->class_opt.size());
-    stats->lanes_per_query = (uint32_t)opt_lanes(ctx->opt, mode, k);
+    // (with size classes: of the options that apply without them)
+    stats->lanes_per_query = (uint32_t)lanes_used(
+        nclouds == 1 && ctx->class_opt.empty() ? one_cloud_args(a) : a, mode == RTNN_MODE_KNN,
+        opt_lanes(ctx->opt, mode, k), tile_points(ctx));
     fill_stats(ctx, stats);
   }
   return RTNN_OK;

@@ -140,6 +140,9 @@ hipError_t bucket_snap(float* qradius, uint32_t nq, float snap_r, float r, hipSt
 hipError_t launch_search(const SearchArgs& a, int knn_mode, int group_lanes, hipStream_t st,
                          int num_cus, bool wide = true, int tiled = 0, bool deep = false,
                          int pool = 0);
+// Lanes per query of the kernel that launch_search (without `pool`) takes: 1 for
+// the matrix kernel, which takes a query per lane.
+int lanes_used(const SearchArgs& a, bool knn, int group_lanes, int tiled);
 // ---- matrix.hip
 // Range search or KNN (k <= 32) over raster grids by 64 queries per wave, the
 // distances filtered on the matrix cores (one block per tile; no device-resident

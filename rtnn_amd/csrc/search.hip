@@ -1175,6 +1175,16 @@ static bool matrix_rule(const SearchArgs& a, bool knn, int group_lanes, int tile
   return a.tiles || (a.nq >= 1u << 19 && a.nq >= a.near_pts / 2);
 }
 
+// Batches of KNN rows of more than 32 keys at one lane per query.
+static bool long_rows_rule(const SearchArgs& a, bool knn, int group_lanes) {
+  return knn && a.tiles && group_lanes == 1 && a.k > 32 && a.nlevels == 0;
+}
+
+int lanes_used(const SearchArgs& a, bool knn, int group_lanes, int tiled) {
+  if (matrix_rule(a, knn, group_lanes, tiled)) return 1;
+  return long_rows_rule(a, knn, group_lanes) ? 16 : group_lanes;
+}
+
 hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hipStream_t st,
                          int num_cus, bool wide, int tiled, bool deep, int pool) {
   SearchArgs a = a0;
@@ -1217,7 +1227,7 @@ hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hi
   // KNN of longer rows in batches: 16 lanes each, where one lane each inserts
   // every hit of its wave one by one (200 lattices, K = 48: 358 us against
   // 2272; with r = 0.6, far more hits than K, 3.7 ms against 14.9).
-  if (knn_mode && a.tiles && group_lanes == 1 && k > 32 && a.nlevels == 0) {
+  if (long_rows_rule(a, knn_mode != 0, group_lanes)) {
     group_lanes = 16;
     tiled = 0;
   }
