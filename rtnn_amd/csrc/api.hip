@@ -994,6 +994,26 @@ int arm_overflow(rtnn_ctx ctx, uint64_t nq, SearchArgs& a) {
   return RTNN_OK;
 }
 
+// Has the device choose between the matrix and the group kernel for a launch that
+// matrix_rule gives to the former, unless the queries are the points themselves and
+// there is one for two cells or more (consecutive ones are neighbours then).
+int arm_matrix(rtnn_ctx ctx, SearchArgs& a, bool knn, int lanes, int tiled) {
+  if (!matrix_rule(a, knn, lanes, tiled)) return RTNN_OK;
+  if (a.queries == a.spts && 2 * ctx->n >= ctx->ncells) return RTNN_OK;
+  const int re = ensure_reduction(ctx);
+  if (re) return re;
+  uint32_t* head = ctx->bbox_tmp.as<uint32_t>();  // the ticket, then the choice
+  CK(matrix_probe(a, knn, ctx->bbox_tmp.as<float>() + 64, head, head + 1,
+                  static_cast<uint32_t*>(ctx->pbbox.p) + 12, ctx->st));
+  a.gate = head + 1;
+  return RTNN_OK;
+}
+// Lanes per query of a's kernel, once the launch has ended.
+int lanes_taken(rtnn_ctx ctx, const SearchArgs& a, bool knn, int lanes, int tiled) {
+  if (a.gate && static_cast<uint32_t*>(ctx->pbbox.p)[12] != 0) return lanes;
+  return lanes_used(a, knn, lanes, tiled);
+}
+
 void fill_stats(rtnn_ctx ctx, rtnn_stats* s) {
   if (!s) return;
   for (int a = 0; a < 3; ++a) s->grid_dims[a] = (uint32_t)ctx->hgrid.dim[a];
@@ -1258,6 +1278,9 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
   if (pooled) {
     rc = arm_overflow(ctx, nq, a);
     if (rc) return rc;
+  } else if (!packet) {
+    rc = arm_matrix(ctx, a, mode == RTNN_MODE_KNN, gl, tiled);
+    if (rc) return rc;
   }
   if (packet)
     CK(launch_knn_packet(a, tree, ctx->st, ctx->num_cus));
@@ -1280,7 +1303,7 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
     stats->search_launches = pooled ? 2 : 1;
     stats->lanes_per_query = (uint32_t)(pooled   ? 64 / ctx->opt.queries_per_wave
                                         : packet ? 1
-                                                 : lanes_used(a, mode == RTNN_MODE_KNN, gl, tiled));
+                                                 : lanes_taken(ctx, a, mode == RTNN_MODE_KNN, gl, tiled));
     fill_stats(ctx, stats);
   }
   return RTNN_OK;
@@ -1625,6 +1648,9 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
   if (pooled) {
     rc = arm_overflow(ctx, nq, a);
     if (rc) return rc;
+  } else if (!walk) {
+    rc = arm_matrix(ctx, a, true, gl, tile_points(ctx));
+    if (rc) return rc;
   }
   if (walk && gl == 1)
     CK(launch_knn_packet(a, tree, ctx->st, ctx->num_cus));
@@ -1685,7 +1711,7 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
     stats->search_launches = 2 + (tree_fallback ? 0 : kGrowStages) + (pooled ? 1 : 0);
     stats->lanes_per_query = (uint32_t)(pooled            ? 64 / ctx->opt.queries_per_wave
                                         : walk && gl == 1 ? 1
-                                                          : lanes_used(a, true, gl, tile_points(ctx)));
+                                                          : lanes_taken(ctx, a, true, gl, tile_points(ctx)));
     fill_stats(ctx, stats);
   }
   return RTNN_OK;

@@ -84,6 +84,9 @@ struct SearchArgs {
   // group kernel then searches those rows again.
   uint32_t* ovf_rows;
   uint32_t* ovf_count;
+  // nullable (matrix_probe): where *gate is 0 the matrix kernel takes the queries,
+  // else the group kernel *gate of them (all).
+  const uint32_t* gate;
 };
 
 // Box tree over the Morton-sorted points (packet.hip): leaves of kLeafPts

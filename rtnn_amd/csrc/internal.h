@@ -139,7 +139,9 @@ hipError_t bucket_snap(float* qradius, uint32_t nq, float snap_r, float r, hipSt
 // counter zero on entry).
 hipError_t launch_search(const SearchArgs& a, int knn_mode, int group_lanes, hipStream_t st,
                          int num_cus, bool wide = true, int tiled = 0, bool deep = false,
-                         int pool = 0);
+                         int pool = 0, int per_cu = 8);
+// Whether launch_search (without `pool`) takes the matrix kernel.
+bool matrix_rule(const SearchArgs& a, bool knn, int group_lanes, int tiled);
 // Lanes per query of the kernel that launch_search (without `pool`) takes: 1 for
 // the matrix kernel, which takes a query per lane.
 int lanes_used(const SearchArgs& a, bool knn, int group_lanes, int tiled);
@@ -148,6 +150,11 @@ int lanes_used(const SearchArgs& a, bool knn, int group_lanes, int tiled);
 // distances filtered on the matrix cores (one block per tile; no device-resident
 // query count).  launch_search chooses it.
 hipError_t launch_matrix(const SearchArgs& a, bool knn, hipStream_t st);
+// Whether a's queries lie close enough together for it: *use_groups (for a.gate)
+// and *told (may be pinned host memory) become non-zero where they do not.  part:
+// kBboxPartBytes; *ticket: 0 before and after.
+hipError_t matrix_probe(const SearchArgs& a, bool knn, float* part, uint32_t* ticket,
+                        uint32_t* use_groups, uint32_t* told, hipStream_t st);
 // ---- packet.hip
 // Level layout of the box tree of n points over `box` (2 * boxes float4).
 BoxTree box_tree_layout(uint64_t n, float4* box);

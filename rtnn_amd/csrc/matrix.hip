@@ -105,6 +105,52 @@ __device__ __forceinline__ void emit_row(const SearchArgs& a, const double (&lis
   }
 }
 
+// The cells that a lane's query reaches (none: lo0 > hi0, or lo1 > hi1, ...).
+struct CellBox {
+  int lo0, hi0, lo1, hi1, lo2, hi2;
+  __device__ bool some() const { return lo0 <= hi0 && lo1 <= hi1 && lo2 <= hi2; }
+};
+__device__ __forceinline__ CellBox cell_box(const GridDesc& g, const float4& q, float R) {
+  CellBox c;
+  cell_range(g, q.x, R, 0, c.lo0, c.hi0);
+  cell_range(g, q.y, R, 1, c.lo1, c.hi1);
+  cell_range(g, q.z, R, 2, c.lo2, c.hi2);
+  return c;
+}
+
+// Block of the cells of a group of queries: those of `todo` near lane `lead`.
+struct Block {
+  uint32_t b0, b1, b2, e0, ny, rows;
+};
+__device__ __forceinline__ bool near_lead(const CellBox& c, int lead) {
+  const int f0 = __builtin_amdgcn_readlane(c.lo0, lead);
+  const int f1 = __builtin_amdgcn_readlane(c.lo1, lead);
+  const int f2 = __builtin_amdgcn_readlane(c.lo2, lead);
+  return abs(c.lo0 - f0) <= kSpanX && abs(c.lo1 - f1) <= kSpanYZ && abs(c.lo2 - f2) <= kSpanYZ;
+}
+__device__ __forceinline__ Block block_of(const CellBox& c, bool in) {
+  Block b;
+  b.b0 = wave_min_u32(in ? (uint32_t)c.lo0 : ~0u);
+  b.b1 = wave_min_u32(in ? (uint32_t)c.lo1 : ~0u);
+  b.b2 = wave_min_u32(in ? (uint32_t)c.lo2 : ~0u);
+  b.e0 = wave_max_u32(in ? (uint32_t)c.hi0 : 0u);
+  b.ny = wave_max_u32(in ? (uint32_t)c.hi1 : 0u) - b.b1 + 1u;
+  b.rows = b.ny * (wave_max_u32(in ? (uint32_t)c.hi2 : 0u) - b.b2 + 1u);
+  return b;
+}
+// Points s .. e of the block's row of cells j (none past the last row).
+__device__ __forceinline__ void row_run(const SearchArgs& a, const GridDesc& g, const Block& b,
+                                        uint32_t j, uint32_t& s, uint32_t& e) {
+  s = 0;
+  e = 0;
+  if (j < b.rows) {
+    const uint32_t rowc = g.cell_base + ((b.b2 + j / b.ny) * (uint32_t)g.dim[1] + b.b1 +
+                                         j % b.ny) * (uint32_t)g.dim[0];
+    s = a.cell_start[rowc + b.b0];
+    e = a.cell_start[rowc + b.e0 + 1u];
+  }
+}
+
 template <int KC, bool KNN>
 __global__ __launch_bounds__(kTileQ)
 __attribute__((amdgpu_waves_per_eu(MatCfg<KC>::kOccupancy))) void k_topk_matrix(
@@ -123,6 +169,7 @@ __attribute__((amdgpu_waves_per_eu(MatCfg<KC>::kOccupancy))) void k_topk_matrix(
   const uint32_t mine = (((uint32_t)lane >> 2) & 1u) * 16u + (((uint32_t)lane >> 3) & 3u) * 4u +
                         ((uint32_t)lane & 3u);
   const double none = key_empty();
+  if (a.gate && *a.gate != 0) return;
   uint32_t q0, q1, gi;
   tile_of(a, a.nq, xcd_swizzle(blockIdx.x, gridDim.x), q0, q1, gi);
   const uint32_t qi = q0 + threadIdx.x;
@@ -135,11 +182,8 @@ __attribute__((amdgpu_waves_per_eu(MatCfg<KC>::kOccupancy))) void k_topk_matrix(
   const float R = active ? query_radius(a, qi, qs) : a.r;
   const float R2 = R * R;
   float lim = r2_limit(R2);
-  int lo0, hi0, lo1, hi1, lo2, hi2;
-  cell_range(g, qv.x, R, 0, lo0, hi0);
-  cell_range(g, qv.y, R, 1, lo1, hi1);
-  cell_range(g, qv.z, R, 2, lo2, hi2);
-  bool todo = active && lo0 <= hi0 && lo1 <= hi1 && lo2 <= hi2;
+  const CellBox cells = cell_box(g, qv, R);
+  bool todo = active && cells.some();
 
   const uint32_t base = a.local_index ? g.point_base : 0u;
   double list[KC];
@@ -198,29 +242,21 @@ __attribute__((amdgpu_waves_per_eu(MatCfg<KC>::kOccupancy))) void k_topk_matrix(
   bool in = false, all = false;
   float cx = 0.f, cy = 0.f, cz = 0.f;
   float bx = 0.f, by = 0.f, bz = 0.f, one = 0.f, c0 = 0.f, c1 = 0.f;
-  uint32_t b0 = 0, b1 = 0, b2 = 0, e0 = 0, ny = 1, rows = 0, rb = 0;
+  Block blk{0, 0, 0, 0, 1, 0};
+  uint32_t rb = 0;
   uint32_t s = 0, e = 0, p0 = 0, p1 = 0;
   uint64_t runs = 0;
   bool last = false;
 #pragma unroll 1
   while (!last) {
-    if (rb >= rows && runs == 0 && p0 == p1) {
+    if (rb >= blk.rows && runs == 0 && p0 == p1) {
       // The queries near the first one left, the block of their cells.
       const uint64_t left = __ballot(todo);
       if (left != 0) {
         const int lead = __builtin_ctzll(left);
-        const int f0 = __builtin_amdgcn_readlane(lo0, lead);
-        const int f1 = __builtin_amdgcn_readlane(lo1, lead);
-        const int f2 = __builtin_amdgcn_readlane(lo2, lead);
-        in = todo && abs(lo0 - f0) <= kSpanX && abs(lo1 - f1) <= kSpanYZ &&
-             abs(lo2 - f2) <= kSpanYZ;
+        in = todo && near_lead(cells, lead);
         todo = todo && !in;
-        b0 = wave_min_u32(in ? (uint32_t)lo0 : ~0u);
-        b1 = wave_min_u32(in ? (uint32_t)lo1 : ~0u);
-        b2 = wave_min_u32(in ? (uint32_t)lo2 : ~0u);
-        e0 = wave_max_u32(in ? (uint32_t)hi0 : 0u);
-        ny = wave_max_u32(in ? (uint32_t)hi1 : 0u) - b1 + 1u;
-        rows = ny * (wave_max_u32(in ? (uint32_t)hi2 : 0u) - b2 + 1u);
+        blk = block_of(cells, in);
         rb = 0;
         cx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(qv.x), lead));
         cy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(qv.y), lead));
@@ -253,16 +289,8 @@ __attribute__((amdgpu_waves_per_eu(MatCfg<KC>::kOccupancy))) void k_topk_matrix(
     while (cnt < kCap) {
       if (p0 == p1) {
         if (runs == 0) {
-          if (rb >= rows) break;
-          const uint32_t j = rb + (uint32_t)lane;
-          s = 0;
-          e = 0;
-          if (j < rows) {
-            const uint32_t rowc = g.cell_base + ((b2 + j / ny) * (uint32_t)g.dim[1] + b1 +
-                                                 j % ny) * (uint32_t)g.dim[0];
-            s = a.cell_start[rowc + b0];
-            e = a.cell_start[rowc + e0 + 1u];
-          }
+          if (rb >= blk.rows) break;
+          row_run(a, g, blk, rb + (uint32_t)lane, s, e);
           rb += kWave;
           runs = __ballot(e > s);
           continue;
@@ -336,6 +364,140 @@ __attribute__((amdgpu_waves_per_eu(MatCfg<KC>::kOccupancy))) void k_topk_matrix(
   }
 
   emit_row<KC, KNN>(a, list, active, row, qs, R);
+}
+
+// Whether the queries suit this kernel, from up to 1024 waves spread over all:
+// *use_groups becomes a.nq where groups of lanes are the better, 0 where it is
+// (*told, which may be pinned host memory, 1 or 0).
+//
+// What decides is how many groups a wave's queries fall into, how many points
+// these list and how many one query tests alone.  A wave of queries unlike the
+// points (uniform ones over clumps, sparse ones on a fine grid) lists many for
+// few tests, and the few waves that list the most are alone on the chip in the
+// end.  The weights are fitted, in ns per wave, to 146 searches of 0.6 to 2
+// million queries (uniform points, sphere surfaces, Gaussian clusters, Levy
+// flights; queries as the points or uniform over their box).  The probe and the
+// other kernel's empty launch take 12 us; with them the slowest choice takes 1.44
+// times the faster kernel alone (queries mostly outside the points' box), the
+// others at most 1.3 (searches of 50 us) and 1.15 from 200 us on.  By this kernel
+// always, as by counts of points and queries alone, it was up to 9.5 times: 1M
+// uniform queries over a Levy flight of 2M points, r = 2, K = 8, 469 us by groups,
+// 4461 by this kernel, 487 with the probe.
+constexpr int kProbeBlocks = 256, kProbeMaxGroups = 16;
+constexpr int kProbeSums = 4;  // groups, listed points, their squares, own points
+struct ProbeWeights {
+  float group, listed, heaviest, base, own;
+};
+
+__global__ __launch_bounds__(kTileQ) void k_matrix_probe(const SearchArgs a, const ProbeWeights pw,
+                                                         float* __restrict__ part,
+                                                         uint32_t* __restrict__ ticket,
+                                                         uint32_t* __restrict__ use_groups,
+                                                         uint32_t* __restrict__ told) {
+  __shared__ float s_v[kMatWaves][kProbeSums];
+  __shared__ uint32_t s_last;
+  const int w = (int)threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  const uint32_t waves = (uint32_t)(((uint64_t)a.nq + kWave - 1) / kWave);
+  const uint32_t probes = min(waves, (uint32_t)(kProbeBlocks * kMatWaves));
+  const uint32_t me = blockIdx.x * kMatWaves + (uint32_t)w;
+  float v[kProbeSums] = {};
+  if (me < probes) {
+    const uint32_t qi = (uint32_t)((uint64_t)me * waves / probes) * kWave + (uint32_t)lane;
+    const bool active = qi < a.nq;
+    const GridDesc g = a.grids[0];
+    const float4 qv = active ? a.queries[qi] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float R = active ? query_radius(a, qi, qi) : a.r;
+    const CellBox c = cell_box(g, qv, R);
+    const bool some = active && c.some();
+    bool todo = some;
+    float listed = 0.0f, own = 0.0f;
+    int groups = 0;
+    for (uint64_t left = __ballot(todo); left != 0 && groups < kProbeMaxGroups;
+         left = __ballot(todo), ++groups) {
+      const bool in = todo && near_lead(c, __builtin_ctzll(left));
+      todo = todo && !in;
+      const Block b = block_of(c, in);
+      for (uint32_t j = (uint32_t)lane; j < b.rows; j += kWave) {
+        uint32_t s, e;
+        row_run(a, g, b, j, s, e);
+        listed += (float)(e - s);
+      }
+    }
+    // eight of the queries alone, 16 lanes each
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int src = (lane & ~15) + 8 * h + 4;
+      const int w0 = __shfl(c.lo0, src, kWave), w1 = __shfl(c.lo1, src, kWave),
+                w2 = __shfl(c.lo2, src, kWave), x0 = __shfl(c.hi0, src, kWave),
+                x1 = __shfl(c.hi1, src, kWave), x2 = __shfl(c.hi2, src, kWave);
+      const int sy = x1 - w1 + 1;
+      const int rows = __shfl(some ? 1 : 0, src, kWave) * sy * (x2 - w2 + 1);
+      for (int j = lane & 15; j < rows; j += 16) {
+        const uint32_t rowc = g.cell_base + ((uint32_t)(w2 + j / sy) * (uint32_t)g.dim[1] +
+                                             (uint32_t)(w1 + j % sy)) * (uint32_t)g.dim[0];
+        own += (float)(a.cell_start[rowc + x0 + 1] - a.cell_start[rowc + w0]);
+      }
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+      listed += __shfl_xor(listed, o, kWave);
+      own += __shfl_xor(own, o, kWave);
+    }
+    v[0] = (float)groups;
+    v[1] = listed;
+    v[2] = listed * listed;
+    v[3] = own * 0.125f;
+  }
+  if (lane == 0)
+#pragma unroll
+    for (int i = 0; i < kProbeSums; ++i) s_v[w][i] = v[i];
+  __syncthreads();
+  // Folded by the last block to finish, as in k_bbox.
+  if (threadIdx.x == 0) {
+    for (int i = 0; i < kProbeSums; ++i) {
+      float t = 0.0f;
+      for (int u = 0; u < kMatWaves; ++u) t += s_v[u][i];
+      __hip_atomic_store(&part[kProbeSums * blockIdx.x + i], t, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    s_last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+             gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!s_last || w != 0) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll
+  for (int i = 0; i < kProbeSums; ++i) v[i] = 0.0f;
+  for (uint32_t b = (uint32_t)lane; b < gridDim.x; b += kWave)
+#pragma unroll
+    for (int i = 0; i < kProbeSums; ++i)
+      v[i] += __hip_atomic_load(&part[kProbeSums * b + i], __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1)
+#pragma unroll
+    for (int i = 0; i < kProbeSums; ++i) v[i] += __shfl_xor(v[i], o, kWave);
+  if (lane == 0) {
+    const float each = 1.0f / (float)probes;
+    const float here = pw.group * v[0] * each + pw.listed * v[1] * each +
+                       pw.heaviest * v[2] / (fmaxf(v[1], 1.0f) * (float)waves);
+    const bool groups = here > pw.base + pw.own * v[3] * each;
+    *use_groups = groups ? a.nq : 0u;
+    *told = groups ? 1u : 0u;
+    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+hipError_t matrix_probe(const SearchArgs& a, bool knn, float* part, uint32_t* ticket,
+                        uint32_t* use_groups, uint32_t* told, hipStream_t st) {
+  if (a.tiles || a.nq == 0) return hipErrorInvalidValue;
+  static_assert(kProbeBlocks * kProbeSums * 4 <= kBboxPartBytes, "partial sums");
+  const ProbeWeights pw = knn ? ProbeWeights{0.2f, 0.0128f, 3.0f, 4.5f, 0.094f}
+                              : ProbeWeights{2.5f, 0.006f, 30.0f, 12.0f, 0.05f};
+  hipLaunchKernelGGL(k_matrix_probe, dim3(kProbeBlocks), dim3(kTileQ), 0, st, a, pw, part, ticket,
+                     use_groups, told);
+  return hipGetLastError();
 }
 
 template <int KC>

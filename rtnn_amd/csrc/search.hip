@@ -1159,7 +1159,8 @@ uint32_t max_k_for_group(int group_lanes) {
 // at the default 16 lanes per query, KNN at proposed radii with 2 and in batches
 // with one, up to the keys its registers hold.  A wave takes 64 queries, so it wants many of them
 // (graph-captured batches excepted: the group kernel walks those 256 queries at a
-// time) that are neighbours and not much sparser than the points.  Pass time,
+// time) that are not much sparser than the points; whether they are neighbours is
+// measured where the caller does not know (matrix_probe).  Pass time,
 // group / matrix kernel, us: uniform points, r = 2.4, K = 32: 100k 137 / 152,
 // 300k 296 / 206, 1M 855 / 437; r = 1.2 (6 hits a query), K = 8: 300k 170 / 179,
 // 1M 429 / 320; sphere surfaces, K = 32: 1.2M points and 0.3M queries 345 / 409,
@@ -1167,7 +1168,7 @@ uint32_t max_k_for_group(int group_lanes) {
 // (18k points) 152 / 93, 48 167 / 112, 200 341 / 216; KNN of 200, one lane each
 // against it: K = 16 357 / 207, r = 0.3 and K = 32 1443 / 388.  (At 4 lanes and compact
 // buffers, which a tuned program sets, the group kernel is 1.1 times as fast.)
-static bool matrix_rule(const SearchArgs& a, bool knn, int group_lanes, int tiled) {
+bool matrix_rule(const SearchArgs& a, bool knn, int group_lanes, int tiled) {
   if (a.nlevels > 0 || tiled != 0 || a.nq_dev || a.qsel || a.near_pts == 0) return false;
   if (!knn && (group_lanes != 16 || a.k > 32)) return false;
   if (knn && a.tiles && (group_lanes != 1 || a.k > 32)) return false;
@@ -1186,7 +1187,7 @@ int lanes_used(const SearchArgs& a, bool knn, int group_lanes, int tiled) {
 }
 
 hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hipStream_t st,
-                         int num_cus, bool wide, int tiled, bool deep, int pool) {
+                         int num_cus, bool wide, int tiled, bool deep, int pool, int per_cu) {
   SearchArgs a = a0;
   if (a.nq_dev) a.persistent = 1;  // tile count known only on the device
   const uint32_t k = a.k;
@@ -1222,8 +1223,15 @@ hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hi
     return launch_search(o, knn_mode, 4, st, num_cus, true, 0, true, 0);
   }
   if (k == 0 || k > max_k_for_group(group_lanes)) return hipErrorInvalidValue;
-  if (matrix_rule(a, knn_mode != 0, group_lanes, tiled))
-    return launch_matrix(a, knn_mode != 0, st);
+  if (matrix_rule(a, knn_mode != 0, group_lanes, tiled)) {
+    const hipError_t e = launch_matrix(a, knn_mode != 0, st);
+    if (e != hipSuccess || !a.gate) return e;
+    SearchArgs o = a0;
+    o.nq_dev = a0.gate;
+    o.gate = nullptr;
+    // blocks enough to even out clumped points (32 a CU; 8: up to 1.1 times the time)
+    return launch_search(o, knn_mode, group_lanes, st, num_cus, wide, 0, deep, 0, 32);
+  }
   // KNN of longer rows in batches: 16 lanes each, where one lane each inserts
   // every hit of its wave one by one (200 lattices, K = 48: 358 us against
   // 2272; with r = 0.6, far more hits than K, 3.7 ms against 14.9).
@@ -1243,7 +1251,7 @@ hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hi
   if (a.ntiles == 0) return hipSuccess;
   uint32_t blocks = a.ntiles;
   if (a.persistent) {
-    uint32_t cap = (uint32_t)(num_cus > 0 ? num_cus : 256) * 8u;
+    uint32_t cap = (uint32_t)(num_cus > 0 ? num_cus : 256) * (uint32_t)per_cu;
     if (blocks > cap) blocks = cap;
   }
   const dim3 grid(blocks);
