@@ -13,7 +13,6 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
-#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -22,13 +21,13 @@
 #include <mutex>
 #include <set>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "../../include/rtnn_hip.h"
 #include "common.h"
 #include "internal.h"
 #include "mlp.h"
+#include "staged.h"
 
 // Allocation statistics of the library (all contexts of the process): the
 // reference's memstatlib (src/memstatlib/memstatlib.cpp:10-32) interposes
@@ -822,27 +821,6 @@ int output_targets(rtnn_ctx ctx, uint64_t nq, uint32_t k, int32_t* out_idx, floa
   return RTNN_OK;
 }
 
-// Device memory to the caller's pageable host memory.  The runtime's own copy
-// moves it at 17 GB/s, one thread copying from a pinned buffer; here chunks
-// travel through a ring of pinned slots (8 to 32 MiB, kept by the context), and
-// threads of this call, started while the search still runs, copy each from its
-// slot as it lands.  Each chunk costs the queue about 20 us, each thread copies
-// about 12 GB/s.  Search and copy of 61 MB of rows: 3424 -> 1588 us (1 MiB
-// chunks 2138; 6 or 8 threads no better), 410 MB: 23.5 -> 9.4 ms, 16 MB: 1044 ->
-// 582 us, 8 MB: 552 -> 392, 5 MB: 395 -> 308; below 4 MB the threads' start
-// costs what they win.
-struct HostPiece {
-  void* dst;
-  const void* src;
-  uint64_t bytes;
-};
-constexpr int kCopySlots = 8, kCopyDepth = 3, kCopyThreads = 4;
-constexpr uint64_t kStagedBytes = 4ull << 20;
-
-uint64_t copy_slot_bytes(uint64_t total) {
-  return std::min<uint64_t>(4ull << 20,
-                            std::max<uint64_t>(1ull << 20, (total / 8 + 65535) & ~65535ull));
-}
 // The ring and its events; false (use the runtime's copy) if they cannot be had.
 bool ensure_ring(rtnn_ctx ctx, uint64_t total) {
   hipError_t e = ctx->pcopy.ensure(kCopySlots * copy_slot_bytes(total));
@@ -852,88 +830,15 @@ bool ensure_ring(rtnn_ctx ctx, uint64_t total) {
   return e == hipSuccess;
 }
 
-int copy_staged(rtnn_ctx ctx, const HostPiece* piece, int npieces, uint64_t total) {
-  const uint64_t slot_bytes = copy_slot_bytes(total);
-  uint64_t first[3] = {0, 0, 0};  // first chunk of each piece
-  for (int i = 0; i < npieces; ++i)
-    first[i + 1] = first[i] + (piece[i].bytes + slot_bytes - 1) / slot_bytes;
-  const uint64_t chunks = first[npieces];
-  char* const slots = static_cast<char*>(ctx->pcopy.p);
-  auto chunk = [&](uint64_t j) {
-    const int i = npieces > 1 && j >= first[1] ? 1 : 0;
-    const uint64_t off = (j - first[i]) * slot_bytes;
-    return HostPiece{static_cast<char*>(piece[i].dst) + off,
-                     static_cast<const char*>(piece[i].src) + off,
-                     std::min(slot_bytes, piece[i].bytes - off)};
-  };
-  auto unload = [&](uint64_t j) {
-    const HostPiece c = chunk(j);
-    std::memcpy(c.dst, slots + (j % kCopySlots) * slot_bytes, c.bytes);
-  };
-  // Chunk j is thread (j mod threads)'s, in order: it waits until `landed`
-  // passes j.  A slot is free again once its chunk's thread has passed it.
-  std::atomic<uint64_t> landed{0};
-  std::atomic<uint64_t> passed[kCopyThreads];  // chunks each thread has copied
-  for (auto& x : passed) x.store(0);
-  std::atomic<bool> stop{false};
-  int nth = 0;
-  std::thread th[kCopyThreads];
-  auto work = [&](int w, int of) {
-    for (uint64_t j = (uint64_t)w; j < chunks; j += (uint64_t)of) {
-      while (landed.load(std::memory_order_acquire) <= j) {
-        if (stop.load(std::memory_order_relaxed)) return;
-        std::this_thread::yield();
-      }
-      unload(j);
-      passed[w].fetch_add(1, std::memory_order_release);
-    }
-  };
-  // The threads sleep until the first chunk has landed (the search may take
-  // long), then poll.  of: how many of them there are.
-  std::mutex mu;
-  std::condition_variable cv;
-  bool go = false;
-  int of = 1;
-  auto start = [&](int w) {
-    {
-      std::unique_lock<std::mutex> lk(mu);
-      cv.wait(lk, [&] { return go; });
-    }
-    work(w, of);
-  };
-  auto release = [&] {
-    std::lock_guard<std::mutex> lk(mu);
-    of = nth > 0 ? nth : 1;
-    go = true;
-    cv.notify_all();
-  };
-  try {
-    for (; nth < kCopyThreads; ++nth) th[nth] = std::thread(start, nth);
-  } catch (...) {  // as many as there are; none: this thread copies
-  }
-  hipError_t e = hipSuccess;
-  uint64_t sent = 0;
-  for (uint64_t j = 0; j < chunks && e == hipSuccess; ++j) {
-    for (; sent < chunks && sent < j + kCopyDepth && e == hipSuccess; ++sent) {
-      if (sent >= kCopySlots && nth > 0) {  // the slot's last chunk: o
-        const uint64_t o = sent - kCopySlots;
-        while (passed[o % nth].load(std::memory_order_acquire) <= o / nth) std::this_thread::yield();
-      }
-      const HostPiece c = chunk(sent);
-      e = hipMemcpyAsync(slots + (sent % kCopySlots) * slot_bytes, c.src, c.bytes,
-                         hipMemcpyDeviceToHost, ctx->st);
-      if (e == hipSuccess) e = hipEventRecord(ctx->ev_slot[sent % kCopySlots], ctx->st);
-    }
-    if (e == hipSuccess) e = hipEventSynchronize(ctx->ev_slot[j % kCopySlots]);
-    if (e != hipSuccess) break;
-    if (nth == 0) unload(j);
-    landed.store(j + 1, std::memory_order_release);
-    if (j == 0) release();
-  }
-  if (e != hipSuccess) stop.store(true);
-  release();
-  for (int w = 0; w < nth; ++w) th[w].join();
-  CK(e);
+int copy_pieces(rtnn_ctx ctx, const HostPiece* piece, int npieces, uint64_t total) {
+  CK((hipError_t)rtnn::copy_staged(
+      piece, npieces, total, ctx->pcopy.p,
+      [&](int slot, void* dst, const void* src, uint64_t bytes) {
+        const hipError_t e =
+            hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->st);
+        return (int)(e == hipSuccess ? hipEventRecord(ctx->ev_slot[slot], ctx->st) : e);
+      },
+      [&](int slot) { return (int)hipEventSynchronize(ctx->ev_slot[slot]); }));
   return RTNN_OK;
 }
 
@@ -954,7 +859,7 @@ int copy_out(rtnn_ctx ctx, uint64_t nq, uint32_t k, int32_t* out_idx, float* out
   const int np = out_d2 ? 2 : 1;
   if (np * bytes >= kStagedBytes && pageable(out_idx) && (!out_d2 || pageable(out_d2)) &&
       ensure_ring(ctx, np * bytes))
-    return copy_staged(ctx, piece, np, np * bytes);
+    return copy_pieces(ctx, piece, np, np * bytes);
   for (int i = 0; i < np; ++i)
     CK(hipMemcpyAsync(piece[i].dst, piece[i].src, bytes, hipMemcpyDeviceToHost, ctx->st));
   return RTNN_OK;
