@@ -60,9 +60,9 @@ typedef struct {
   uint32_t max_cells;     /* cap on grid cells (cell edge grows to respect it)      */
   int   grid_levels;      /* learned/partitioned KNN: 1 = one raster grid of edge
                              r / cell_factor; >= 2 = hierarchical Morton grid with
-                             that many levels (edges r, r/2, ...), or with one lane
-                             per query (queries_per_wave 0 or 64, k <= 64) the
-                             packet walk over a box tree; 0 = auto (learned 1,
+                             that many levels (edges r, r/2, ...), or for k <= 64
+                             the packet walk over a box tree (one lane per query,
+                             whatever queries_per_wave); 0 = auto (learned 1,
                              partitioned 5)                                       */
   float level_alpha;      /* hierarchical: a query of radius R walks the finest
                              level whose cell edge is >= R * level_alpha (0: 1.0) */
@@ -92,10 +92,10 @@ typedef struct {
                              and do not fall back; 0 = the network alone        */
   int   tree_lanes;       /* no effect any more (that walk takes one lane per
                              query); checked (0, 1, 2, 4 or 8)                  */
-  int   tree_fallback;    /* hierarchical-grid KNN (k <= 64), the packet walk:
-                             0 = the rows short at their proposed radius are
-                             searched once more at r; 1 = through the radius-
-                             growth stages (as on raster grids)               */
+  int   tree_fallback;    /* learned KNN by the packet walk: 0 = every query is
+                             searched at r at once; 1 = at its proposed radius,
+                             short rows through the radius-growth stages (as on
+                             raster grids)                                    */
 } rtnn_options;
 
 /* Filled by search entry points when a non-NULL pointer is passed. */
@@ -182,10 +182,10 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
  * points gives a launch radius min(r, sqrt(3)*(iter+1)*cell); a query whose
  * sphere holds fewer than k hits is searched again at a grown radius (up to
  * four growth stages, then r; a row searched at r is final), so the result
- * equals rtnn_search(..., RTNN_MODE_KNN, ...).  With one lane per query on a
- * hierarchical grid (the default) the packet walk takes the place of the launch
- * radius: every query is searched at r, bounded from its first leaves on by the
- * k-th nearest point found so far, so no row is short. */
+ * equals rtnn_search(..., RTNN_MODE_KNN, ...).  For k <= 64 on a hierarchical grid
+ * (the default) the packet walk takes the place of the launch radius: every query
+ * is searched at r, bounded from its first leaves on by the k-th nearest point
+ * found so far, so no row is short. */
 int rtnn_search_partitioned(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
                             float r, uint32_t k,
                             int32_t* out_idx, float* out_d2, int out_on_device,
@@ -219,7 +219,8 @@ int rtnn_mlp_set_weights(rtnn_ctx ctx, const float* blob /* RTNN_MLP_NBLOB */);
 
 /* KNN where the MLP proposes r' <= r per query; queries with fewer than k hits
  * within r' (stats->fallback_queries) are searched again at grown radii and
- * finally at r, so the result equals rtnn_search(..., RTNN_MODE_KNN, ...). */
+ * finally at r, so the result equals rtnn_search(..., RTNN_MODE_KNN, ...).  The
+ * packet walk (grid_levels >= 2, k <= 64, tree_fallback 0) searches at r at once. */
 int rtnn_search_learned(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
                         float r, uint32_t k,
                         int32_t* out_idx, float* out_d2, int out_on_device,

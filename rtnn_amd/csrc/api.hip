@@ -683,10 +683,8 @@ int build_hgrid(rtnn_ctx ctx, float r, int want_levels) {
     CK(cell_bounds(ctx->keys.as<uint32_t>(), n, (uint32_t)(1ull << (3 * (b - l))),
                    ctx->cell_start.as<uint32_t>() + lv[l].cell_base, ctx->tmp.as<uint32_t>(),
                    ctx->st, 3 * l));
-  // The box tree of the packet walk, which searches the short rows.
-  CK(ctx->boxes.ensure(32 * box_tree_layout(n, nullptr).boxes));
-  CK(build_box_tree(ctx->pts.as<float>(), ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(),
-                    box_tree_layout(n, ctx->boxes.as<float4>()), ctx->st));
+  CK(gather_points(ctx->pts.as<float>(), ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(),
+                   ctx->st));
   ctx->ncells = total;
   ctx->spts_current = true;
   ctx->hlevels = L;
@@ -1470,13 +1468,15 @@ int compute_proposals(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t n
 }
 
 // The proposals of a search that walks packets: the box tree and the queries in
-// its order; the MLP's radii from the counts of the edge-r cells (the cells of
-// the hierarchical grid's top level).  The density partition needs no radii
-// here: they would bound a query's sphere by a cube that holds k points, and the
-// walk, which starts from the leaves around the query, is bounded by the k-th
-// point found so far.  Its rows are searched at r and none falls short (Gaussian
-// mixture, 1M, K = 8: radii and their level tables took 0.45 ms of a pass).
-int packet_proposals(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq, int on_device,
+// its order.  Radii only with tree_fallback = 1, the MLP's (from the counts of the
+// edge-r cells, the cells of the hierarchical grid's top level): the walk starts
+// from the leaves around the query and is bounded by the k-th point found so far,
+// so a smaller radius saves it little, and a second walk for the short rows, which
+// are not neighbours any more, costs more than the first (learned KNN, 1M points
+// and queries, K = 16: uniform points, r = 2, 1849 us at proposed radii, 720 at r;
+// sphere surfaces, r = 10, 1477 / 722).  Searched at r, no row falls short.  (The
+// density partition's radii and level tables took 0.45 ms of a pass of 1M.)
+int packet_proposals(rtnn_ctx ctx, bool proposes, const float* qxyz, uint64_t nq, int on_device,
                      float r, const float4** qproc, BoxTree* tree) {
   int rc = build_packet_tree(ctx, tree);
   if (rc) return rc;
@@ -1484,7 +1484,7 @@ int packet_proposals(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq
   if (rc) return rc;
   CK(hipEventRecord(ctx->ev[1], ctx->st));
   CK(ctx->qradius.ensure(4 * nq));
-  if (kind != Proposal::kLearned) return RTNN_OK;
+  if (!proposes) return RTNN_OK;
   rc = build_count_grid(ctx, r, false, true);
   if (rc) return rc;
   CK(mlp_propose(ctx->mlp, *qproc, (uint32_t)nq, ctx->pgrid.as<GridDesc>(), false,
@@ -1517,19 +1517,17 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
   CK(hipSetDevice(ctx->device));
   CK(hipEventRecord(ctx->ev[0], ctx->st));
   const float4* qproc = nullptr;
-  // One query per lane on a hierarchical grid: the packet walk over the box
-  // tree, which needs no level tables (learned_cap does: it takes the
-  // partition's radii from them).
+  // A hierarchical grid and k <= 64: the packet walk over the box tree, whatever the
+  // lanes asked for; it needs no level tables.
   const int gl = group_lanes_from_opt(ctx, RTNN_MODE_KNN, k);
   BoxTree tree{};
-  const bool packet = proposal_levels(ctx, kind) >= 2 && gl == 1 && k <= 64 &&
-                      !pool_requested(ctx, k) &&
-                      !(kind == Proposal::kLearned && ctx->opt.learned_cap != 0);
-  rc = packet ? packet_proposals(ctx, kind, qxyz, nq, on_device, r, &qproc, &tree)
+  const bool packet = proposal_levels(ctx, kind) >= 2 && k <= 64;
+  if (packet && (gl < 0 || k > max_k_for_group(gl)) && !pool_requested(ctx, k))
+    return fail(ctx, RTNN_ERR_UNSUPPORTED, "k=%u not supported by the selected kernel", k);
+  const bool proposes = !packet || (kind == Proposal::kLearned && ctx->opt.tree_fallback != 0);
+  rc = packet ? packet_proposals(ctx, proposes, qxyz, nq, on_device, r, &qproc, &tree)
               : compute_proposals(ctx, kind, qxyz, nq, on_device, r, k, &qproc);
   if (rc) return rc;
-  if (ctx->hlevels > 0) tree = box_tree_layout(ctx->n, ctx->boxes.as<float4>());
-  const bool walk = packet || ctx->hlevels > 0;  // `tree` stands over spts
   CK(hipEventRecord(ctx->ev[2], ctx->st));
   OutBufs o;
   rc = output_targets(ctx, nq, k, out_idx, out_d2, out_on_device, o);
@@ -1541,23 +1539,23 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
   uint32_t* hits[2] = {lists[0] + 2 * nq, lists[0] + 3 * nq};
   uint32_t* counters = lists[0] + 4 * nq;
   CK(fill_u32(counters, kGrowStages + 1, 0, ctx->st));
-  const bool pooled = pool_requested(ctx, k) && ctx->hlevels == 0;
-  if (!pooled && (gl < 0 || k > max_k_for_group(gl)))
+  const bool pooled = pool_requested(ctx, k) && !packet && ctx->hlevels == 0;
+  if (!packet && !pooled && (gl < 0 || k > max_k_for_group(gl)))
     return fail(ctx, RTNN_ERR_UNSUPPORTED, "k=%u not supported by the selected kernel", k);
   // Stage 1: every query at its proposed radius r'.
   SearchArgs a = base_args(ctx, qproc, nq, r, k, o);
-  a.qradius = packet && kind == Proposal::kPartition ? nullptr : ctx->qradius.as<float>();
+  a.qradius = proposes ? ctx->qradius.as<float>() : nullptr;
   a.short_rows = lists[0];
   a.short_count = &counters[0];
   a.short_hits = hits[0];
   if (pooled) {
     rc = arm_overflow(ctx, nq, a);
     if (rc) return rc;
-  } else if (!walk) {
+  } else if (!packet) {
     rc = arm_matrix(ctx, a, true, gl, tile_points(ctx));
     if (rc) return rc;
   }
-  if (walk && gl == 1)
+  if (packet)
     CK(launch_knn_packet(a, tree, ctx->st, ctx->num_cus));
   else
     CK(launch_search(a, 1, gl, ctx->st, ctx->num_cus, wide_buffers(ctx), tile_points(ctx), false,
@@ -1575,7 +1573,7 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
   // not its radius, bounds it -- so its short rows go straight to the last
   // stage (option tree_fallback = 1: through the growth stages, which the
   // autotuner tries).
-  const bool tree_fallback = walk && k <= 64 && ctx->opt.tree_fallback == 0;
+  const bool tree_fallback = packet && ctx->opt.tree_fallback == 0;
   for (int j = tree_fallback ? kGrowStages : 0; j <= kGrowStages; ++j) {
     SearchArgs s = base_args(ctx, qproc, nq, r, k, o);
     s.qsel = tree_fallback ? lists[0] : lists[j & 1];
@@ -1590,7 +1588,7 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
     }
     // Beyond k = 64 (the register top-k and the 4-lane buffers) the rows go
     // to 16- or 64-lane groups.
-    if (walk && k <= 64) {
+    if (packet) {
       CK(launch_knn_packet(s, tree, ctx->st, ctx->num_cus));
       continue;
     }
@@ -1614,9 +1612,9 @@ int proposal_search(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t nq,
     stats->ms_total = ev_ms(ctx->ev[0], ctx->ev[5]);
     stats->fallback_queries = nshort;
     stats->search_launches = 2 + (tree_fallback ? 0 : kGrowStages) + (pooled ? 1 : 0);
-    stats->lanes_per_query = (uint32_t)(pooled            ? 64 / ctx->opt.queries_per_wave
-                                        : walk && gl == 1 ? 1
-                                                          : lanes_taken(ctx, a, true, gl, tile_points(ctx)));
+    stats->lanes_per_query = (uint32_t)(pooled   ? 64 / ctx->opt.queries_per_wave
+                                        : packet ? 1
+                                                 : lanes_taken(ctx, a, true, gl, tile_points(ctx)));
     fill_stats(ctx, stats);
   }
   return RTNN_OK;
@@ -2602,13 +2600,8 @@ int rtnn_autotune(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device, i
   if (k <= 64)
     for (int i = 0; i < ncf; ++i)
       for (int qpw : {16, 32, 64}) cands.push_back({cfs[i], qpw, plain ? 0 : 1, 0.0f, 3, 0});
-  // Hierarchical grids: the packet walk (one lane per query), which does not
-  // depend on the levels, and 4-lane groups on the level rule.
-  if (!plain) {
-    cands.push_back({0.0f, 0, 5, 0.0f, 0, 0});
-    for (int lv : {3, 5})
-      for (float al : {1.0f, 0.5f}) cands.push_back({0.0f, 16, lv, al, 0, 0});
-  }
+  // Hierarchical grids: the packet walk, which does not depend on the levels.
+  if (!plain) cands.push_back({0.0f, 0, 5, 0.0f, 0, 0});
   for (const Cand& cand : cands) {
     {
       const int qpw = cand.qpw;

@@ -1114,9 +1114,13 @@ static void launch_group(const SearchArgs& a, bool knn, bool wide, int tile, dim
       return;
     }
   }
-  if (knn && hier)
-    hipLaunchKernelGGL((k_topk_group<G, KB, true, true, true>), grid, dim3(kTileQ), 0, st, a);
-  else if (knn && wide)
+  if constexpr (KB > 64) {  // shorter rows take the packet walk
+    if (hier) {
+      hipLaunchKernelGGL((k_topk_group<G, KB, true, true, true>), grid, dim3(kTileQ), 0, st, a);
+      return;
+    }
+  }
+  if (knn && wide)
     hipLaunchKernelGGL((k_topk_group<G, KB, true, false, true>), grid, dim3(kTileQ), 0, st, a);
   else if (knn)
     hipLaunchKernelGGL((k_topk_group<G, KB, true, false, false>), grid, dim3(kTileQ), 0, st, a);
@@ -1239,8 +1243,8 @@ hipError_t launch_search(const SearchArgs& a0, int knn_mode, int group_lanes, hi
     group_lanes = 16;
     tiled = 0;
   }
-  // hierarchical grids: KNN by groups (one lane per query is the packet walk's)
-  if (a.nlevels > 0 && (group_lanes == 1 || !knn_mode)) return hipErrorInvalidValue;
+  // hierarchical grids: KNN rows of more than 64 keys (others are the packet walk's)
+  if (a.nlevels > 0 && (k <= 64 || !knn_mode)) return hipErrorInvalidValue;
   if (!a.tiles) {
     // Implicit tiles: a block of the thread kernel takes kTileQ queries, a
     // block of the group kernel one query per group, so small workloads still
