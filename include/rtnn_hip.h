@@ -149,7 +149,9 @@ int rtnn_search(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
 /* Stream-ordered form of rtnn_search for device-resident queries (qxyz, or
  * NULL for the points) and outputs: the grid build, query ordering and search
  * are enqueued on `stream` (a hipStream_t) and the call returns without
- * waiting.  The work is ordered after the context's earlier calls, and the
+ * waiting for it.  (The first KNN of these with default lanes after
+ * rtnn_set_points, or with another radius, waits for one kernel that measures how
+ * the points lie, on a stream of its own.)  The work is ordered after the context's earlier calls, and the
  * context's later calls are ordered after it (event waits between the two
  * streams), so the context may be used again at once; the caller synchronises
  * `stream` before reading the outputs.  Replaces the reference's per-batch
