@@ -104,10 +104,16 @@ void k_topk_thread(const SearchArgs a) {
       if (rr + 1 < nrows) row_bounds(rr + 1, s_next, e_next);
       for (uint32_t j0 = s; j0 < e; j0 += kUnroll) {
         // kUnroll loads in flight before the first test: unconditional loads
-        // (a slot past the run reloads its last point and is not tested).
+        // (a slot past the run reloads its last point and is not tested), issued in
+        // the order of the tests, each of which then waits for its own only (left
+        // to itself the scheduler put the first one last: 476 -> 492 us for 1M
+        // uniform queries, K = 16).
         float4 pv[kUnroll];
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) pv[u] = a.spts[min(j0 + (uint32_t)u, e - 1)];
+        for (int u = 0; u < kUnroll; ++u) {
+          pv[u] = a.spts[min(j0 + (uint32_t)u, e - 1)];
+          __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
           if (j0 + u >= e) break;
