@@ -265,9 +265,9 @@ struct rtnn_ctx_s {
   hipEvent_t ev[8] = {};
   hipEvent_t ev_join = nullptr;  // orders rtnn_search_async work with the context stream
   // The query ordering runs on st2 while the point grid is sorted on st:
-  // ev_desc (grid descriptors uploaded) starts it, ev_q joins it back.
+  // ev_build (the build starts) starts it, ev_q joins it back.
   hipStream_t st2 = nullptr;
-  hipEvent_t ev_desc = nullptr, ev_q = nullptr;
+  hipEvent_t ev_build = nullptr, ev_q = nullptr;
   DevBuf tmp2;  // radix-sort scratch of the query ordering
 
   // radius proposals (learned / partitioned)
@@ -333,7 +333,7 @@ struct rtnn_ctx_s {
     for (auto& e : ev)
       if (e) (void)hipEventDestroy(e);
     if (ev_join) (void)hipEventDestroy(ev_join);
-    if (ev_desc) (void)hipEventDestroy(ev_desc);
+    if (ev_build) (void)hipEventDestroy(ev_build);
     if (ev_q) (void)hipEventDestroy(ev_q);
     tmp2.release();
     if (st2) (void)hipStreamDestroy(st2);
@@ -627,9 +627,10 @@ int probe_cells_async(rtnn_ctx ctx, float r, uint64_t nq, uint32_t k, int* lanes
   return RTNN_OK;
 }
 
-// Builds the grid of plan_single.  desc_event: separate queries follow, ordered
-// on the second stream as soon as the descriptor is on the device.
-int build_grid(rtnn_ctx ctx, float cell, bool desc_event = true) {
+// Builds the grid of plan_single.  own_queries: separate queries follow, ordered
+// on the second stream meanwhile.
+int build_grid(rtnn_ctx ctx, float cell, bool own_queries = true) {
+  if (own_queries) CK(hipEventRecord(ctx->ev_build, ctx->st));
   GridDesc g;
   const int rp = plan_single(ctx, cell, g);
   if (rp) return rp;
@@ -649,7 +650,6 @@ int build_grid(rtnn_ctx ctx, float cell, bool desc_event = true) {
     CK(cell_count_single(ctx->pts.as<float>(), n, ctx->hgrid, ctx->grids.as<GridDesc>(),
                          ctx->counts.as<uint32_t>(), ctx->keys.as<uint32_t>(),
                          ctx->vals.as<uint32_t>(), ctx->st));
-    if (desc_event) CK(hipEventRecord(ctx->ev_desc, ctx->st));
     CK(cell_scan_place(ctx->pts.as<float>(), n, ctx->ncells, ctx->counts.as<uint32_t>(),
                        ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(),
                        ctx->cell_start.as<uint32_t>(), ctx->tmp.as<uint32_t>(),
@@ -662,7 +662,6 @@ int build_grid(rtnn_ctx ctx, float cell, bool desc_event = true) {
     // pageable copy, which costs the host more than a launch).
     CK(cell_keys_single(ctx->pts.as<float>(), n, ctx->hgrid, ctx->grids.as<GridDesc>(),
                         ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), ctx->st));
-    if (desc_event) CK(hipEventRecord(ctx->ev_desc, ctx->st));
     CK(radix_sort_pairs(ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), n,
                         bits_for(ctx->ncells - 1), ctx->tmp.as<uint32_t>(), ctx->st,
                         &ctx->sort_passes));
@@ -683,6 +682,7 @@ int build_grid(rtnn_ctx ctx, float cell, bool desc_event = true) {
 // same sorted keys.  Level tables larger than 2^27 cells are skipped (queries
 // use the finest built level).
 int build_hgrid(rtnn_ctx ctx, float r, int want_levels) {
+  CK(hipEventRecord(ctx->ev_build, ctx->st));
   int L = std::max(2, std::min(want_levels, 8));
   float c0 = 0, inv0 = 0;
   int b = 0;
@@ -726,7 +726,6 @@ int build_hgrid(rtnn_ctx ctx, float r, int want_levels) {
   CK(ctx->grids.ensure(sizeof(GridDesc) * L));
   CK(hipMemcpyAsync(ctx->grids.p, lv.data(), sizeof(GridDesc) * L, hipMemcpyHostToDevice,
                     ctx->st));
-  CK(hipEventRecord(ctx->ev_desc, ctx->st));
   CK(ctx->keys.ensure(4 * n));
   CK(ctx->vals.ensure(4 * n));
   CK(ctx->cell_start.ensure(4 * total));
@@ -754,6 +753,7 @@ int build_hgrid(rtnn_ctx ctx, float r, int want_levels) {
 // grid of 2^10 cells per axis over their box (the order only decides how
 // compact the boxes are, never a result).  *t describes it.
 int build_packet_tree(rtnn_ctx ctx, BoxTree* t) {
+  CK(hipEventRecord(ctx->ev_build, ctx->st));
   const uint64_t n = ctx->n;
   GridDesc g;
   std::memset(&g, 0, sizeof g);
@@ -778,7 +778,6 @@ int build_packet_tree(rtnn_ctx ctx, BoxTree* t) {
   *t = box_tree_layout(n, ctx->boxes.as<float4>());
   CK(cell_keys_single(ctx->pts.as<float>(), n, ctx->hgrid, ctx->grids.as<GridDesc>(),
                       ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), ctx->st));
-  CK(hipEventRecord(ctx->ev_desc, ctx->st));
   CK(radix_sort_pairs(ctx->keys.as<uint32_t>(), ctx->vals.as<uint32_t>(), n, 3 * kPacketKeyBits,
                       ctx->tmp.as<uint32_t>(), ctx->st, &ctx->sort_passes));
   CK(build_box_tree(ctx->pts.as<float>(), ctx->vals.as<uint32_t>(), n, ctx->spts.as<float4>(), *t,
@@ -792,8 +791,9 @@ constexpr int kQueryKeyBits = 8;  // Morton bits per axis of the query order
 
 // Prepares queries in processing order (float4 with the output row in w).
 // Returns the processing-order array through *qproc.  The ordering runs on
-// ctx->st2, started by ctx->ev_desc (recorded by the grid build once its
-// descriptors are on the device), so it overlaps the point sort on ctx->st;
+// ctx->st2, started by ctx->ev_build (recorded as the grid build starts; the grid's
+// descriptor comes by value), so it overlaps that build on ctx->st: started only
+// after the build's first kernel, the counting of 1M points, it ended 36 us later;
 // ctx->st waits for it before returning work that reads *qproc.  always_order:
 // the packet walk of the proposal methods, which needs neighbours in a wave.
 int prepare_queries(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
@@ -808,7 +808,7 @@ int prepare_queries(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
   CK(ctx->tmp2.ensure(4 * radix_tmp_words(nq)));
   if (!on_device) CK(ctx->qin.ensure(12 * nq));
   hipStream_t s2 = ctx->st2;
-  CK(hipStreamWaitEvent(s2, ctx->ev_desc, 0));
+  CK(hipStreamWaitEvent(s2, ctx->ev_build, 0));
   const float* dq = qxyz;
   if (!on_device) {
     CK(hipMemcpyAsync(ctx->qin.p, qxyz, 12 * nq, hipMemcpyHostToDevice, s2));
@@ -823,7 +823,7 @@ int prepare_queries(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
     int maxdim = std::max(ctx->hgrid.dim[0], std::max(ctx->hgrid.dim[1], ctx->hgrid.dim[2]));
     const int bits = bits_for((uint64_t)(maxdim - 1));
     const int shift = std::max(0, bits - key_bits);
-    CK(query_morton_keys(dq, nq, ctx->grids.as<GridDesc>(), shift, ctx->qkeys.as<uint32_t>(),
+    CK(query_morton_keys(dq, nq, ctx->hgrid, nullptr, shift, ctx->qkeys.as<uint32_t>(),
                          ctx->qvals.as<uint32_t>(), s2));
     CK(radix_sort_pairs(ctx->qkeys.as<uint32_t>(), ctx->qvals.as<uint32_t>(), nq,
                         3 * std::min(bits, key_bits), ctx->tmp2.as<uint32_t>(), s2,
@@ -1036,7 +1036,7 @@ int rtnn_create(int device, rtnn_ctx* out) {
   }
   for (auto& ev : c->ev) (void)hipEventCreate(&ev);
   (void)hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming);
-  (void)hipEventCreateWithFlags(&c->ev_desc, hipEventDisableTiming);
+  (void)hipEventCreateWithFlags(&c->ev_build, hipEventDisableTiming);
   (void)hipEventCreateWithFlags(&c->ev_q, hipEventDisableTiming);
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
@@ -1373,7 +1373,7 @@ int rtnn_search_noalloc(rtnn_ctx ctx, const float* xyz, uint64_t n, const float*
     if (ctx->opt.query_order == 1) {
       CK(iota_u32(qvals, nq, st));
     } else {
-      CK(query_morton_keys(qxyz, nq, grid, -1, qkeys, qvals, st));
+      CK(query_morton_keys(qxyz, nq, GridDesc{}, grid, -1, qkeys, qvals, st));
       CK(radix_sort_pairs(qkeys, qvals, nq, 3 * kQueryKeyBits, tmp, st, nullptr));
     }
     CK(gather_points(qxyz, qvals, nq, qs, st));

@@ -940,13 +940,15 @@ hipError_t gather_points(const float* xyz, const uint32_t* vals, uint64_t n, flo
   return hipGetLastError();
 }
 
+// The grid by value, or (grid not null) planned on the device.
 __global__ __launch_bounds__(256) void k_query_morton(const float* __restrict__ q, uint64_t nq,
+                                                      const GridDesc gv,
                                                       const GridDesc* __restrict__ grid,
                                                       int shift, uint32_t* __restrict__ keys,
                                                       uint32_t* __restrict__ vals) {
   uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= nq) return;
-  const GridDesc g = *grid;
+  const GridDesc g = grid ? *grid : gv;
   if (shift < 0) {
     // Grid planned on the device: 8 Morton bits per axis of the widest
     // axis's cell coordinate (the host's rule for a known grid).
@@ -962,11 +964,11 @@ __global__ __launch_bounds__(256) void k_query_morton(const float* __restrict__ 
   vals[i] = (uint32_t)i;
 }
 
-hipError_t query_morton_keys(const float* q, uint64_t nq, const GridDesc* g, int shift,
-                             uint32_t* keys, uint32_t* vals, hipStream_t st) {
+hipError_t query_morton_keys(const float* q, uint64_t nq, const GridDesc& g, const GridDesc* gdev,
+                             int shift, uint32_t* keys, uint32_t* vals, hipStream_t st) {
   if (nq == 0) return hipSuccess;
   hipLaunchKernelGGL(k_query_morton, dim3((uint32_t)((nq + 255) / 256)), dim3(256), 0, st, q,
-                     nq, g, shift, keys, vals);
+                     nq, g, gdev, shift, keys, vals);
   return hipGetLastError();
 }
 
