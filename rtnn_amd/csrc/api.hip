@@ -441,8 +441,18 @@ int group_lanes_from_opt(rtnn_ctx ctx, int mode, uint32_t k) {
 // 200k 31 / 50, 800k 63 / 95, 1.6M 106 / 124; sphere surfaces (8 cells per
 // point): 200k 32 / 64, 800k 84 / 110, 1.6M 155 / 154.  (10M points, 7 cells
 // each: 1390 against 780.)
-bool count_cells_rule(uint64_t n, uint64_t ncells) {
-  return n <= (1ull << 20) && ncells <= (1ull << 25);
+//
+// What counting loses is the input order inside a cell.  One lane per query (the
+// lanes of a wave walk together where consecutive queries are neighbours) pays for
+// that on ordered points in full cells: range search of a lattice of 100k points,
+// K = 50, 27 points a cell: 1394 us sorted, 1675 counted; 3.4 a cell: 386 / 371; a
+// batch of 200 lattices, 8 a cell: 2018 / 2353.  (Unordered points, 100k uniform,
+// 6.4 a cell: 345 / 307.)  In batches four lanes do so from about a tile (256
+// queries) a cell on (216: 1821 / 1946).  full: points per cell, on average, from
+// which that order is kept.
+constexpr double kNeverFull = 1e300, kFullOneLane = 7.0, kFullFewLanes = 64.0;
+bool count_cells_rule(uint64_t n, uint64_t ncells, double full) {
+  return n <= (1ull << 20) && ncells <= (1ull << 25) && (double)n <= full * (double)ncells;
 }
 
 // Makes the first ncells words of ctx->counts zero for a grid build.  The build
@@ -628,8 +638,8 @@ int probe_cells_async(rtnn_ctx ctx, float r, uint64_t nq, uint32_t k, int* lanes
 }
 
 // Builds the grid of plan_single.  own_queries: separate queries follow, ordered
-// on the second stream meanwhile.
-int build_grid(rtnn_ctx ctx, float cell, bool own_queries = true) {
+// on the second stream meanwhile.  full: of count_cells_rule.
+int build_grid(rtnn_ctx ctx, float cell, bool own_queries = true, double full = kNeverFull) {
   if (own_queries) CK(hipEventRecord(ctx->ev_build, ctx->st));
   GridDesc g;
   const int rp = plan_single(ctx, cell, g);
@@ -642,7 +652,7 @@ int build_grid(rtnn_ctx ctx, float cell, bool own_queries = true) {
   CK(ctx->vals.ensure(4 * n));
   CK(ctx->cell_start.ensure(4 * (ctx->ncells + 1)));
   CK(ctx->spts.ensure(16 * std::max<uint64_t>(n, 1) + kSptsPadBytes));
-  if (count_cells_rule(n, ctx->ncells)) {
+  if (count_cells_rule(n, ctx->ncells, full)) {
     CK(ctx->tmp.ensure(4 * cell_scan_tmp_words(ctx->ncells)));
     const uint64_t zero = ctx->counts_zero;
     const int rc = clear_counts(ctx, ctx->ncells);
@@ -1223,7 +1233,9 @@ static int search_impl(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_devi
       tiled = 0;
     }
   }
-  rc = packet ? build_packet_tree(ctx, &tree) : build_grid(ctx, r / f, qxyz != nullptr);
+  // (the cells that probe_cells gives one lane are not full)
+  const double full = mode == RTNN_MODE_RADIUS && gl == 1 && !pooled ? kFullOneLane : kNeverFull;
+  rc = packet ? build_packet_tree(ctx, &tree) : build_grid(ctx, r / f, qxyz != nullptr, full);
   if (rc) return rc;
   if (timing) CK(hipEventRecord(ctx->ev[1], ctx->st));
   const float4* qproc = nullptr;
@@ -1476,14 +1488,17 @@ int compute_proposals(rtnn_ctx ctx, Proposal kind, const float* qxyz, uint64_t n
   const float f = ctx->opt.cell_factor > 0 ? ctx->opt.cell_factor
                                            : (kind == Proposal::kLearned ? 2.0f : 4.0f);
   const int levels = proposal_levels(ctx, kind);
+  const double full = group_lanes_from_opt(ctx, RTNN_MODE_KNN, k) == 1 && !pool_requested(ctx, k)
+                          ? kFullOneLane
+                          : kNeverFull;
   bool hier = levels >= 2;
-  int rc = hier ? build_hgrid(ctx, r, levels) : build_grid(ctx, r / f);
+  int rc = hier ? build_hgrid(ctx, r, levels) : build_grid(ctx, r / f, true, full);
   if (rc == RTNN_ERR_UNSUPPORTED && hier) {
     // The Morton grid needs the box within 1024 top-level cells of edge r per
     // axis; a wider box (or a smaller r) takes the raster grid, which grows
     // its cell edge to fit the cell budget.
     hier = false;
-    rc = build_grid(ctx, r / f);
+    rc = build_grid(ctx, r / f, true, full);
   }
   if (rc) return rc;
   const float4* qproc = nullptr;
@@ -2210,8 +2225,29 @@ std::vector<float> batched_cells(rtnn_ctx ctx, const uint64_t* offsets, uint32_t
   return v;
 }
 
+// Lanes per query of options o for (mode, k).
+int opt_lanes(const rtnn_options& o, int mode, uint32_t k) {
+  const int qpw = o.queries_per_wave;
+  return qpw > 0 ? 64 / qpw : default_group_lanes(mode, k);
+}
+
+// `full` of count_cells_rule for a batch: its fewest lanes per query, one of them
+// only where the thread kernel takes them.
+double batched_full(rtnn_ctx ctx, uint32_t nclouds, int mode, uint32_t k) {
+  double full = kNeverFull;
+  for (size_t j = 0; j < std::max<size_t>(1, ctx->class_opt.size()); ++j) {
+    const rtnn_options& o = ctx->class_opt.empty() ? ctx->opt : ctx->class_opt[j];
+    const int lanes = opt_lanes(o, mode, k);
+    if (lanes == 1 && (mode == RTNN_MODE_RADIUS || nclouds == 1 || o.lds_tile != 0))
+      full = std::min(full, kFullOneLane);
+    else if (lanes > 1 && lanes <= 4)
+      full = std::min(full, kFullFewLanes);
+  }
+  return full;
+}
+
 int build_batched(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets, uint32_t nclouds,
-                  const std::vector<float>& cells) {
+                  const std::vector<float>& cells, double full = kNeverFull) {
   const uint64_t n = offsets[nclouds];
   // Per-cloud bbox on the device, plan on the host.
   CK(ctx->offs.ensure(8 * (nclouds + 1)));
@@ -2262,7 +2298,7 @@ int build_batched(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets, uint3
   CK(ctx->spts.ensure(16 * n + kSptsPadBytes));
   ctx->spts_current = false;  // spts now holds the clouds, not ctx->pts
   ctx->hlevels = 0;           // and grids/cell_start the clouds' raster grids
-  if (count_cells_rule(n, total)) {
+  if (count_cells_rule(n, total, full)) {
     CK(ctx->tmp.ensure(4 * cell_scan_tmp_words(total)));
     const uint64_t zero = ctx->counts_zero;
     const int rc = clear_counts(ctx, total);
@@ -2310,12 +2346,6 @@ int build_batched(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets, uint3
                     ctx->st));
   ctx->batch_tiles = (uint32_t)tl.size();
   return RTNN_OK;
-}
-
-// Lanes per query of options o for (mode, k).
-int opt_lanes(const rtnn_options& o, int mode, uint32_t k) {
-  const int qpw = o.queries_per_wave;
-  return qpw > 0 ? 64 / qpw : default_group_lanes(mode, k);
 }
 
 // A batch of one cloud: implicit tiles over all its points.
@@ -2504,7 +2534,8 @@ int batched_impl(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets, uint32
   if (timing) CK(hipEventRecord(ctx->ev[0], ctx->st));
   const float f = ctx->opt.cell_factor > 0 ? ctx->opt.cell_factor : default_cell_factor(mode);
   rc = build_batched(ctx, xyz, offsets, nclouds,
-                     batched_cells(ctx, offsets, nclouds, mode, r, r / f));
+                     batched_cells(ctx, offsets, nclouds, mode, r, r / f),
+                     batched_full(ctx, nclouds, mode, k));
   if (rc) return rc;
   if (timing) CK(hipEventRecord(ctx->ev[1], ctx->st));
 
@@ -2974,6 +3005,7 @@ struct rtnn_graph_s {
   uint64_t n = 0;
   uint32_t nclouds = 0, ntiles = 0;
   uint64_t cap_cells = 0;
+  bool counted = false;  // raster grids built by counting (count_cells_rule)
   // Options at capture: the whole batch's, or one per size class with the
   // class-major tile ranges class_tiles[j] .. [j+1].
   rtnn_options opt;
@@ -3036,7 +3068,7 @@ hipError_t enqueue_batched(rtnn_graph g, const float* xyz, float cell, int mode,
   if ((e = plan_batched(g->bboxes.as<float>(), off, g->nclouds, cell, cells, g->cap_cells,
                         g->grids.as<GridDesc>(), status, st)) != hipSuccess)
     return e;
-  if (count_cells_rule(g->n, g->cap_cells)) {
+  if (g->counted) {
     if ((e = cell_count(xyz, g->n, g->grids.as<GridDesc>(), off, g->nclouds,
                         g->counts.as<uint32_t>(), keys, vals, st)) != hipSuccess)
       return e;
@@ -3121,7 +3153,10 @@ int rtnn_graph_batched(rtnn_ctx ctx, const float* xyz, const uint64_t* offsets,
   CK(g->vals.ensure(4 * n));
   CK(g->cell_start.ensure(4 * (g->cap_cells + 1)));
   CK(g->spts.ensure(16 * n + kSptsPadBytes));
-  if (count_cells_rule(n, g->cap_cells)) {
+  // (full cells as the data lies now)
+  g->counted = count_cells_rule(n, g->cap_cells, kNeverFull) &&
+               count_cells_rule(n, ctx->ncells, batched_full(ctx, nclouds, mode, k));
+  if (g->counted) {
     CK(g->tmp.ensure(4 * cell_scan_tmp_words(g->cap_cells)));
     // zero once; every run leaves them zero
     CK(g->counts.ensure(4 * ((g->cap_cells + 3) & ~3ull)));
