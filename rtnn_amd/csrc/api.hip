@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -532,16 +533,26 @@ int plan_single(rtnn_ctx ctx, float cell, GridDesc& g) {
 //       K = 64   mean 2.4          1661 / 2512 / 351 / 436; mean 12  2415 / 8625 / 689 / 826
 //                mean 33           2349 / 10768 / 14788 / 3921
 //       K = 8    clusters, mean 7   489 / 1175 / 1609 / 1366
+// and, packets / one lane (700k points; 1.5M; * without the probe, 15 us):
+//   K = 4   mean 18   391 / 337; 622 / 594     K = 8   mean 18   443 / 457*; 736 / 802*
+//   K = 16  mean 5    480 / 391; 786 / 728             mean 6.5  500 / 490*; 804 / 848*
+//           a lattice, jittered by 2%, mean 4.7  461 / 286; 729 / 510;
+//                                      mean 6.8  472 / 393*; 762 / 665*
+constexpr double kMostMean = 64.0;  // beyond it, packets
+constexpr uint64_t kFewQueries = 1ull << 14;
+constexpr uint32_t kFewDraws = 1u << 14;
 int knn_cell_lanes(uint64_t nq, uint32_t k, double mean, double skew) {
-  if (nq <= 1ull << 14) return mean <= 64.0 ? 16 : 0;
+  if (nq <= kFewQueries) return mean <= kMostMean ? 16 : 0;
   if (skew > 3.0) return 0;
   if (nq <= 1ull << 17) return mean <= 3.0 ? 4 : mean <= 24.0 ? 16 : 0;
-  if (k <= 8) return mean <= 16.0 ? 1 : 0;
-  if (k <= 16) return mean <= 4.0 ? 4 : mean <= 8.0 && nq <= 1ull << 19 ? 16 : 0;
+  if (k <= 8) return mean <= (k <= 4 ? 20.0 : 16.0) ? 1 : 0;
+  if (k <= 16) {
+    if (mean <= 4.0) return 4;
+    return nq <= 1ull << 19 ? (mean <= 8.0 ? 16 : 0) : mean <= 6.0 ? 1 : 0;
+  }
   if (k <= 32) return mean <= 8.0 ? 4 : mean <= 12.0 ? 16 : 0;
   return mean <= 12.0 ? 4 : mean <= 20.0 ? 16 : 0;
 }
-constexpr double kMostMean = 64.0;  // beyond it knn_cell_lanes is 0
 
 // What k_cell_spread is to count for the cells of edge r: false where there is
 // nothing to (no such grid, or so few cells that even evenly spread points would be
@@ -552,11 +563,13 @@ struct SpreadPlan {
   int tbits;    // counters: 2^tbits words
   bool hashed;
 };
-bool plan_spread(rtnn_ctx ctx, float r, SpreadPlan& p) {
+bool plan_spread(rtnn_ctx ctx, float r, uint64_t nq, SpreadPlan& p) {
   if (plan_single(ctx, r, p.g)) return false;
   const uint64_t ncells = grid_cells(p.g);
   if ((double)ctx->n > kMostMean * (double)ncells) return false;
-  p.m = (uint32_t)std::min<uint64_t>(ctx->n, kSpreadDraws);
+  // (few queries ask only whether a cell holds more than kMostMean: 1M points,
+  // 10,000 queries, 197 -> 165 us a pass)
+  p.m = (uint32_t)std::min<uint64_t>(ctx->n, nq <= kFewQueries ? kFewDraws : kSpreadDraws);
   p.tbits = std::max(12, bits_for(8ull * p.m - 1));
   p.hashed = ncells > (1ull << p.tbits);
   return true;
@@ -584,23 +597,40 @@ void spread_stats(const SpreadPlan& p, uint64_t n, const CellSpread& s, double* 
   *skew = cube / (*mean * *mean);
 }
 
+// Waits for the sums of a cell_spread on st.  They are in pinned memory as the
+// kernel ends, some us before the stream says so: large point sets, whose build keeps
+// the queue busy from here on, look for them there (1.5M points, K = 8: 390 -> 370 us
+// a pass; 300k: 150 -> 141), the runtime waits if they do not come soon and reports
+// what went wrong.  Small calls would lose up to 10 us to the unfinished stream.
+int await_spread(rtnn_ctx ctx, const CellSpread* s, hipStream_t st) {
+  if (ctx->n > 1ull << 18) {
+    const auto t0 = std::chrono::steady_clock::now();
+    while (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(1))
+      if (__atomic_load_n(&s->done, __ATOMIC_ACQUIRE) != 0) return RTNN_OK;
+  }
+  CK(hipStreamSynchronize(st));
+  return RTNN_OK;
+}
+
 // Measures the cells of edge r and sets *lanes to knn_cell_lanes; waits for the
 // device (one launch and the wait: about 20 us).
 int probe_cells(rtnn_ctx ctx, float r, uint64_t nq, uint32_t k, int* lanes) {
   *lanes = 0;
   SpreadPlan p;
-  if (!plan_spread(ctx, r, p)) return RTNN_OK;
+  if (!plan_spread(ctx, r, nq, p)) return RTNN_OK;
   const int re = ensure_reduction(ctx);
   if (re) return re;
   const uint64_t words = 1ull << p.tbits, zero = ctx->counts_zero;
   const int rz = clear_counts(ctx, words);
   if (rz) return rz;
   CellSpread* s = static_cast<CellSpread*>(ctx->pbbox.p);
+  s->done = 0;
   CK(cell_spread(ctx->pts.as<float>(), ctx->n, p.m, p.g, p.hashed, p.tbits,
                  ctx->counts.as<uint32_t>(),
                  reinterpret_cast<uint64_t*>(ctx->bbox_tmp.as<uint32_t>() + 64),
                  ctx->bbox_tmp.as<uint32_t>(), s, ctx->st));
-  CK(hipStreamSynchronize(ctx->st));
+  const int rw = await_spread(ctx, s, ctx->st);
+  if (rw) return rw;
   CK(fill_u32(ctx->counts.as<uint32_t>(), words, 0, ctx->st));
   grid_built(ctx, words, zero);
   double mean, skew;
@@ -618,7 +648,7 @@ int probe_cells(rtnn_ctx ctx, float r, uint64_t nq, uint32_t k, int* lanes) {
 int probe_cells_async(rtnn_ctx ctx, float r, uint64_t nq, uint32_t k, int* lanes) {
   *lanes = 0;
   SpreadPlan p;
-  if (!plan_spread(ctx, r, p)) return RTNN_OK;
+  if (!plan_spread(ctx, r, ~0ull, p)) return RTNN_OK;  // (kept for any number of queries)
   if (ctx->spread_edge != p.g.cell) {
     if (!ctx->st4) CK(hipStreamCreateWithFlags(&ctx->st4, hipStreamNonBlocking));
     const uint64_t head = 256 + kBboxPartBytes, words = 1ull << p.tbits;
@@ -626,10 +656,12 @@ int probe_cells_async(rtnn_ctx ctx, float r, uint64_t nq, uint32_t k, int* lanes
     CK(ctx->pspread.ensure(sizeof(CellSpread)));
     uint32_t* tmp = ctx->spread_tmp.as<uint32_t>();
     CellSpread* s = static_cast<CellSpread*>(ctx->pspread.p);
+    s->done = 0;
     CK(fill_u32(tmp, head / 4 + words, 0, ctx->st4));
     CK(cell_spread(ctx->pts.as<float>(), ctx->n, p.m, p.g, p.hashed, p.tbits, tmp + head / 4,
                    reinterpret_cast<uint64_t*>(tmp + 64), tmp, s, ctx->st4));
-    CK(hipStreamSynchronize(ctx->st4));
+    const int rw = await_spread(ctx, s, ctx->st4);
+    if (rw) return rw;
     spread_stats(p, ctx->n, *s, &ctx->spread_mean, &ctx->spread_skew);
     ctx->spread_edge = p.g.cell;
   }

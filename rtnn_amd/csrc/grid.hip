@@ -751,8 +751,9 @@ hipError_t cell_count_single(const float* xyz, uint64_t n, const GridDesc& g, Gr
 // table of 2^tbits where that is the smaller, and takes the number of points
 // counted there before it as its rank.  *spread becomes the sums over the draws
 // of rank and of rank (rank - 1) / 2: the pairs and the triples of draws that
-// share a cell.  Random atomics bound it, hence the sample (131,072 draws 10 us,
-// a million points 60); folded by the last block to finish, as in k_bbox.
+// share a cell; then spread->done is 1.  Random atomics bound it, hence the sample
+// (131,072 draws 10 us, a million points 60); folded by the last block to finish,
+// as in k_bbox.
 __global__ __launch_bounds__(256) void k_cell_spread(const float* __restrict__ xyz, uint64_t n,
                                                      uint32_t m, const GridDesc g, bool hashed,
                                                      int tbits, uint32_t* __restrict__ table,
@@ -812,9 +813,10 @@ __global__ __launch_bounds__(256) void k_cell_spread(const float* __restrict__ x
       v[c] += __hip_atomic_load(&part[2 * b + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   fold();
   if (threadIdx.x == 0) {
+    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     spread->pairs = s_sum[0];
     spread->triples = s_sum[1];
-    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&spread->done, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 

@@ -36,6 +36,7 @@ hipError_t bbox(const float* src, float* dst, uint64_t n, float* part, uint32_t*
 constexpr uint32_t kSpreadDraws = 1u << 17;
 struct CellSpread {
   uint64_t pairs, triples;
+  uint32_t done;  // 0 before, 1 once the sums are there
 };
 hipError_t cell_spread(const float* xyz, uint64_t n, uint32_t m, const GridDesc& g, bool hashed,
                        int tbits, uint32_t* table, uint64_t* part, uint32_t* ticket,
