@@ -55,7 +55,9 @@ typedef struct {
   int   queries_per_wave; /* lanes per query = 64 / queries_per_wave: 64 = one query
                              per lane (k <= 64), 32/16/8/4/1 = groups of 2/4/8/16/64
                              lanes (k <= 16/64/64/256/1024); 0 = auto             */
-  int   query_order;      /* 0 auto, 1 input order, 2 Morton order of query cells  */
+  int   query_order;      /* 0 auto, 1 input order, 2 Morton order of query cells; no
+                             effect where learned/partitioned KNN takes the packet
+                             walk (Hilbert order: its queries must be neighbours) */
   int   time_stages;      /* 1: record hipEvent timings into rtnn_stats             */
   uint32_t max_cells;     /* cap on grid cells (cell edge grows to respect it)      */
   int   grid_levels;      /* learned/partitioned KNN: 1 = one raster grid of edge

@@ -368,7 +368,7 @@ int hip_fail(rtnn_ctx c, hipError_t e, const char* what) {
     if (e_ != hipSuccess) return hip_fail(ctx, e_, #expr); \
   } while (0)
 
-constexpr int kPacketKeyBits = 10;  // Morton bits per axis of the packet walk's points
+constexpr int kPacketKeyBits = 10;  // Hilbert bits per axis of the packet walk's points
 
 int bits_for(uint64_t maxval) {
   int b = 0;
@@ -434,7 +434,7 @@ int group_lanes_from_opt(rtnn_ctx ctx, int mode, uint32_t k) {
   return gl;
 }
 
-// Raster grids are built by counting up to a million points, by sorting beyond:
+// Raster grids are built by counting up to 2^20 points, by sorting beyond:
 // the counting build is a third of the launches, which is what a small grid
 // costs, but its atomics on random cells run at about 25 G/s, and its 16-byte
 // stores are scattered where the sort's gather reads are.  Build time by
@@ -442,6 +442,8 @@ int group_lanes_from_opt(rtnn_ctx ctx, int mode, uint32_t k) {
 // 200k 31 / 50, 800k 63 / 95, 1.6M 106 / 124; sphere surfaces (8 cells per
 // point): 200k 32 / 64, 800k 84 / 110, 1.6M 155 / 154.  (10M points, 7 cells
 // each: 1390 against 780.)
+// The line is where counting is ahead on every such set; at 1.6M it is by a sixth
+// of the build or not at all.
 //
 // What counting loses is the input order inside a cell.  One lane per query (the
 // lanes of a wave walk together where consecutive queries are neighbours) pays for
@@ -791,7 +793,7 @@ int build_hgrid(rtnn_ctx ctx, float r, int want_levels) {
   return RTNN_OK;
 }
 
-// Box tree over ctx->pts for the packet walk: points in Morton order of a cubic
+// Box tree over ctx->pts for the packet walk: points in Hilbert order of a cubic
 // grid of 2^10 cells per axis over their box (the order only decides how
 // compact the boxes are, never a result).  *t describes it.
 int build_packet_tree(rtnn_ctx ctx, BoxTree* t) {
@@ -829,7 +831,7 @@ int build_packet_tree(rtnn_ctx ctx, BoxTree* t) {
   return RTNN_OK;
 }
 
-constexpr int kQueryKeyBits = 8;  // Morton bits per axis of the query order
+constexpr int kQueryKeyBits = 8;  // bits per axis of the query order
 
 // Prepares queries in processing order (float4 with the output row in w).
 // Returns the processing-order array through *qproc.  The ordering runs on
@@ -859,9 +861,9 @@ int prepare_queries(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device,
   if (ctx->opt.query_order == 1 && !always_order) {
     CK(iota_u32(ctx->qvals.as<uint32_t>(), nq, s2));
   } else {
-    // Morton order of the query cells, 8 bits per axis (cells merged in
-    // aligned 2^shift blocks on finer grids): 3 radix passes, and a wave's
-    // queries still share their neighbourhood.
+    // Morton order of the query cells (packets: Hilbert order), key_bits per axis
+    // (cells merged in aligned 2^shift blocks on finer grids): at 8 three radix
+    // passes, and a wave's queries still share their neighbourhood.
     int maxdim = std::max(ctx->hgrid.dim[0], std::max(ctx->hgrid.dim[1], ctx->hgrid.dim[2]));
     const int bits = bits_for((uint64_t)(maxdim - 1));
     const int shift = std::max(0, bits - key_bits);
@@ -2709,7 +2711,7 @@ int rtnn_autotune(rtnn_ctx ctx, const float* qxyz, uint64_t nq, int on_device, i
   for (int i = 0; i < ncf; ++i)
     for (int j = 0; j < nqpw; ++j) {
       const bool group = qpws[j] > 0 && qpws[j] < 64;
-      if (plain && !range && !group && i > 0) continue;  // the packet walk has no cells
+      if (plain && !range && !group && i > 0) continue;  // packets have no cells
       cands.push_back({cfs[i], qpws[j], plain ? 0 : 1, 0.0f, group ? 2 : 0, 0});
       if (group) {
         cands.push_back({cfs[i], qpws[j], plain ? 0 : 1, 0.0f, 1, 0});

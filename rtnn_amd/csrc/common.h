@@ -89,7 +89,7 @@ struct SearchArgs {
   const uint32_t* gate;
 };
 
-// Box tree over the Morton-sorted points (packet.hip): leaves of kLeafPts
+// Box tree over the points in Hilbert order (packet.hip): leaves of kLeafPts
 // consecutive points, nodes of kFan children.  Level 0 holds the leaves' boxes
 // (minimum at box[2i], maximum at box[2i + 1]), level l + 1 those of kFan
 // consecutive boxes of level l; the top level has at most kFan.

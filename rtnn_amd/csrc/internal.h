@@ -89,10 +89,9 @@ hipError_t count_sorted(const float4* spts, uint64_t n, const GridDesc* g, uint3
 // spts[j] = (xyz[vals[j]], bits(vals[j])).
 hipError_t gather_points(const float* xyz, const uint32_t* vals, uint64_t n, float4* spts,
                          hipStream_t st);
-// Morton key (10 bits per axis) of each query's cell in grid g (or, where set,
-// *gdev), shifted right
-// by `shift` bits per axis (shift < 0: derived on the device from g's widest
-// axis, keeping 8 bits per axis); vals[i] = i.
+// Morton key (Hilbert key where g.morton == 2) of each query's cell in grid g (or,
+// where set, *gdev), the cell shifted right by `shift` bits per axis (shift < 0:
+// derived on the device from g's widest axis, keeping 8 bits per axis); vals[i] = i.
 hipError_t query_morton_keys(const float* q, uint64_t nq, const GridDesc& g, const GridDesc* gdev,
                              int shift, uint32_t* keys, uint32_t* vals, hipStream_t st);
 hipError_t morton3_codes(const uint32_t* xyz, uint64_t n, uint32_t* codes, hipStream_t st);

@@ -19,8 +19,9 @@
 // (v_min_f64 / v_max_f64, see topk.h).
 //
 // A wave's latency bounds it at the 12 (K <= 16) or 8 waves per CU that its LDS
-// allows: the products take a fifth of it, the loads of the block and the stores
-// of the rows most of the rest.  Rows of 64 keys would need every register there
+// and registers allow (learned KNN of 10M, K = 16: the matrix cores busy 0.14 of
+// the time, VALU issue 0.56, a third of the wave cycles waiting for loads, LDS and
+// stores).  Rows of 64 keys would need every register there
 // is and spill (batches of 1024 clouds, K = 64: 20 ms against the group kernel's
 // 13.6), so k > 32 stays with the groups.  A pass against groups of lanes per
 // query, which test each query's candidates alone: 1M uniform points, r = 2.4,

@@ -10,11 +10,11 @@
 // GELU and the BF16 rounding happen in registers, no LDS transpose.  The last
 // layer (64 -> 1) is a VALU dot product reduced over the four lane groups.
 //
-// Training (k_mlp_grad, k_mlp_adam): FP32 VALU, one sample per lane, the
-// same BF16 rounding of weights and activations in the forward pass as the
-// MFMA path (straight-through gradients to the FP32 master weights).
-// Per-block gradient partials are summed in a fixed order, so training is
-// deterministic.
+// Training (k_mlp_grad, k_mlp_adam): FP32 VALU, a block of 64 samples whose
+// products each lane takes in 4 x 4 tiles of the result, the same BF16 rounding
+// of weights and activations in the forward pass as the MFMA path
+// (straight-through gradients to the FP32 master weights).  Per-block gradient
+// partials are summed in a fixed order, so training is deterministic.
 //
 // GELU is Hendrycks & Gimpel's sigmoid form (2016, "Gaussian Error Linear
 // Units", section 2), x sigma(1.702 x), with the logistic replaced by the

@@ -21,7 +21,7 @@
 // 16 keys into 16 costs about 210 instructions per wave where inserting keys
 // one by one cost about 100 per key with most lanes idle.
 //
-// VALU issue bounds it (0.8 of the slots on sphere surfaces, K = 16).  Against
+// VALU issue bounds it (0.9 of its cycles on sphere surfaces, K = 16).  Against
 // one query per lane over the cells of a grid of edge r (a pass, 1M points and
 // queries): Gaussian mixture r = 20, K = 8: 10.5 -> 0.92 ms, K = 50: 153 ->
 // 3.5; sphere surfaces r = 10, K = 16 (4M): 4.73 -> 2.14; uniform points with
@@ -206,7 +206,7 @@ struct PacketCfg {
   static constexpr int kBuf = kOwn ? 12 : 16;  // keys per lane between merges
   static constexpr int kQueue = kOwn ? 8 : 1;  // leaves waiting per lane
   // Waves per SIMD: what 40 KB of LDS per block and a list of 2 KC registers
-  // leave (K = 16: 128 VGPRs, 136 bytes spilled, 2.19 ms a pass at 4M on sphere
+  // leave (K = 16: 128 VGPRs, 88 bytes of scratch, 2.19 ms a pass at 4M on sphere
   // surfaces against 2.39 at three waves).
   static constexpr int kOccupancy = KC <= 16 ? 4 : KC <= 32 ? 2 : 1;
 };

@@ -1167,9 +1167,9 @@ uint32_t max_k_for_group(int group_lanes) {
 
 // Whether the matrix kernel takes the place of the group kernel: range searches
 // at the default 16 lanes per query, KNN at proposed radii with 2 and in batches
-// with one, up to the keys its registers hold.  A wave takes 64 queries, so it wants many of them
-// (graph-captured batches excepted: the group kernel walks those 256 queries at a
-// time) that are not much sparser than the points; whether they are neighbours is
+// with one, up to the keys its registers hold.  A wave takes 64 queries, so it wants
+// many of them (graph-captured batches excepted: the group kernel walks those 256
+// queries at a time) that are not much sparser than the points; whether they are neighbours is
 // measured where the caller does not know (matrix_probe).  Pass time,
 // group / matrix kernel, us: uniform points, r = 2.4, K = 32: 100k 137 / 152,
 // 300k 296 / 206, 1M 855 / 437; r = 1.2 (6 hits a query), K = 8: 300k 170 / 179,

@@ -149,7 +149,7 @@ __device__ inline void key_cx_inplace(double& a, double& b) {
 }
 
 // Sorts N keys ascending: Batcher's odd-even merge sort of the next power of
-// two, whose missing last keys would be the largest (12 keys: 41
+// two, whose missing last keys would be the largest (12 keys: 42
 // compare-exchanges).  One comparator level per template instance,
 // so that every index is a constant and the keys stay in registers.
 template <int N, int P, int Q>
